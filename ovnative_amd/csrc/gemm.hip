@@ -890,25 +890,26 @@ __device__ __forceinline__ void gemm16_tile(const GemmArgs& a, const int wg) {
         const f32x4 wu0 = *reinterpret_cast<const f32x4*>(&qkv_ws[nr - n0 + 16]);
         const f32x4 wg1 = *reinterpret_cast<const f32x4*>(&qkv_ws[nr - n0 + 32]);
         const f32x4 wu1 = *reinterpret_cast<const f32x4*>(&qkv_ws[nr - n0 + 48]);
-        float h[8];
+        float g[8], u[8], h[8];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          h[e] = silu_up_lane(__fmul_rn(f[t][j][e], wg0[e]), __fmul_rn(f[t + 1][j][e], wu0[e]));
-          h[4 + e] =
-              silu_up_lane(__fmul_rn(f[t + 2][j][e], wg1[e]), __fmul_rn(f[t + 3][j][e], wu1[e]));
+          g[e] = __fmul_rn(f[t][j][e], wg0[e]);
+          u[e] = __fmul_rn(f[t + 1][j][e], wu0[e]);
+          g[4 + e] = __fmul_rn(f[t + 2][j][e], wg1[e]);
+          u[4 + e] = __fmul_rn(f[t + 3][j][e], wu1[e]);
         }
-        float am = 0.f;
+        silu_up_lanes(g, u, h);
+        float am = 0.f, nan = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) am = fmaxf(am, fabsf(h[e]));
+        for (int e = 0; e < 8; ++e) {
+          am = fmaxf(am, fabsf(h[e]));
+          nan = __fadd_rn(nan, h[e]);
+        }
         am = fmaxf(am, __shfl_xor(am, 16));
         am = fmaxf(am, __shfl_xor(am, 32));
+        const bool ok = __all(nan == nan && (am == 0.f || (am >= 0x1p-100f && am <= 0x1p120f)));
         const float qinv = am > 0.f ? __fdiv_rn(127.0f, am) : 0.f;
-        uint32_t c0 = 0, c1 = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          c0 |= (uint32_t)(uint8_t)(int8_t)quant_q(h[e], qinv) << (8 * e);
-          c1 |= (uint32_t)(uint8_t)(int8_t)quant_q(h[4 + e], qinv) << (8 * e);
-        }
+        const uint32_t c0 = quant_pack4(h, qinv, ok), c1 = quant_pack4(h + 4, qinv, ok);
         if (m >= a.M) continue;
         const int64_t col = (int64_t)((n0 + (wn * FN + t) * 16) / 32) * 16;  // h column of the block
         *reinterpret_cast<uint32_t*>(a.hq + act_index(m, col + 4 * q, a.hKp, a.h_tiled)) = c0;
@@ -1362,9 +1363,8 @@ hipError_t launch_gemm(const GemmArgs& a, GemmMode mode, hipStream_t st) {
   // SiLU-fused gate/up (sweep over 128x64 / 128x32 / 64x64 / 64x32 tiles, N =
   // 6144, K = 1024, MI355X): up to M = 512 the 32-row tiles give more
   // wavefronts (M = 128: 8.4 us against 11.4 for 128x64; M = 256: 9.8 against
-  // 11.8 for 64x32 of two wavefronts); from M = 600 the 128x64 tile wins
-  // with cache-hot weights (17.4 against 18.1 for the next).  At 512 < M < 1024
-  // (the LM step, whose weights come cold from HBM) 8-wavefront tiles with the
+  // 11.8 for 64x32 of two wavefronts).  Above, up to the large-M form's 640
+  // rows (the LM step, whose weights come cold from HBM), 8-wavefront tiles with the
   // same 64x32 wavefront tile: 256x64 took 16.0 against 17.4 us for 128x64
   // with cold weights, and 128x128 (half as many L2 re-reads of each weight
   // tile, one per 128 rows) takes the step 2.256 against 2.265 ms for 256x64
@@ -1381,13 +1381,12 @@ hipError_t launch_gemm(const GemmArgs& a, GemmMode mode, hipStream_t st) {
     if (a.Kb % 4 || mode == kDumpBlocks) return hipErrorInvalidValue;
     return launch_cfg16_f16<128, 128, 2, 4, 2, 2, false>(a, mode, st);
   }
+  if (wide_applies(a, mode)) return launch_gemm_wide(a, mode, st);
   if (mode == kSiluQuant) {
     if (a.Kb % 4) return hipErrorInvalidValue;
-    if (M >= 2048) return launch_cfg16_silu<128, 64, 2, 2, 4, 2, false>(a, st);
     if (M <= 128) return launch_cfg16_silu<128, 32, 2, 2, 4, 2, true>(a, st);
     if (M <= 512) return launch_cfg16_silu<64, 32, 1, 2, 4, 2, true>(a, st);
-    if (M < 1024) return launch_cfg16_silu<128, 128, 2, 4, 4, 2, true>(a, st);
-    return launch_cfg16_silu<128, 64, 2, 2, 4, 2, true>(a, st);
+    return launch_cfg16_silu<128, 128, 2, 4, 4, 2, true>(a, st);  // below 640 (wide_applies)
   }
   // kDumpBlocks takes the tile the store and residual modes take for the same
   // shape (the kernel differs only after the block products)
