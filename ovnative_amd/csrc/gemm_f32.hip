@@ -20,6 +20,8 @@
 // fragments (row tile, k step) row-tile-major; rows padded to a multiple of 128
 // and k to a multiple of 16, with zeros (activations: rows past M are
 // whatever the producer left, and only ever reach outputs that are not stored).
+#include <type_traits>
+
 #include "gemm.h"
 #include "ovh_common.h"
 
@@ -130,6 +132,59 @@ __global__ __launch_bounds__(256) void f32_split_rows_kernel(int64_t M, int64_t 
   }
 }
 
+// Rows of 256 P columns (P <= 4, 16-byte aligned): one wavefront per row holds
+// the row in registers (one pass over it), four rows per workgroup, and the
+// planes go through LDS so that the four rows' 16-byte slots leave as 64
+// contiguous bytes (a row's own stores are 16 bytes in every 512).  M = 600,
+// K = 1024: 7.8 -> 3.6 us.  Rows past M are left alone (see above).
+template <int P>
+__global__ __launch_bounds__(256) void f32_split_rows_p_kernel(int64_t M,
+                                                               const float* __restrict__ A,
+                                                               _Float16* __restrict__ hi,
+                                                               _Float16* __restrict__ lo,
+                                                               float* __restrict__ scale) {
+  constexpr int cols = 256 * P, Ks = 16 * P, kGroup = 4 * 16 + 16;  // bytes per 8-k group, padded
+  __shared__ __attribute__((aligned(16))) char tile[2][32 * P * kGroup];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t r0 = (int64_t)blockIdx.x * 4, r = r0 + wave;
+  f32x4 x[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p)
+    x[p] = *reinterpret_cast<const f32x4*>(A + (r < M ? r : M - 1) * cols + 256 * p + 4 * lane);
+  float am = 0.f;
+#pragma unroll
+  for (int p = 0; p < P; ++p)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) am = fmaxf(am, fabsf(x[p][e]));
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) am = fmaxf(am, __shfl_xor(am, o));
+  const int ex = pow2_exponent(am);
+  const float inv = ldexpf(1.f, -ex);
+  if (lane == 0 && r < M) scale[r] = ldexpf(1.f, ex);
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    h4 vh, vl;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      _Float16 a, b;
+      split_scaled(x[p][e], inv, a, b);
+      vh[e] = a;
+      vl[e] = b;
+    }
+    const int at = (32 * p + (lane >> 1)) * kGroup + wave * 16 + (lane & 1) * 8;
+    *reinterpret_cast<h4*>(&tile[0][at]) = vh;
+    *reinterpret_cast<h4*>(&tile[1][at]) = vl;
+  }
+  __syncthreads();
+  // slot c: 8-k group c / 4 of row c % 4
+  for (int c = threadIdx.x; c < 2 * 128 * P; c += 256) {
+    const int plane = c >= 128 * P, d = c - plane * 128 * P, g = d >> 2, rr = d & 3;
+    if (r0 + rr < M)
+      *reinterpret_cast<h8*>((plane ? lo : hi) + plane_index(r0 + rr, 8 * g, Ks)) =
+          *reinterpret_cast<const h8*>(&tile[plane][g * kGroup + rr * 16]);
+  }
+}
+
 // The final RMSNorm of the LM (rmsnorm_f32, cpp/src/backend/cpu/ops_cpu.cpp:
 // 38-62, the same sum of squares as rmsnorm_quantize: eight fma chains, element
 // i into chain i % 8, chains added 0..7; xn = (x * scale) * w) for rows of 256*P
@@ -204,90 +259,151 @@ __global__ __launch_bounds__(64) void rmsnorm_split_rows_kernel(const float* __r
 }
 
 // ---------------------------------------------------------------------------
-// The GEMM: 128 x 128 output tiles (weight columns n x activation rows m), four
-// wavefronts of 64 x 64 (2 x 2 MFMA tiles of 32 x 32); one 16-k step per LDS
-// stage (8 weight and 8 activation fragments, 16 KiB), moved by
-// global_load_lds_dwordx4 (each wavefront 4 fragments per stage) through an
-// NST-stage ring, each wavefront waiting on its own DMA count; XCD-aware tile
-// order (an XCD walks a contiguous range of weight column tiles).
-
+// The GEMM: output tiles of 128 weight columns n x BM activation rows m, four
+// wavefronts of 64 x BM/2 (2 x BM/64 MFMA tiles of 32 x 32); one 16-k step per
+// LDS stage (8 weight and BM/16 activation fragments), moved by
+// global_load_lds_dwordx4 through an NST-stage ring, each wavefront waiting on
+// its own DMA count.  What bounds it: the LDS port (a step of the 128-row tile
+// moves 48 KB, 384 clocks at 128 bytes, beside 384 clocks of products) and
+// power (the f16 matrix core on real data with fragment reads runs at 1.5 of
+// its 2.5 PFLOP/s).  So stage s + 1's fragments are read into a second register
+// set between the products of stage s, one read after each product; stage s's
+// slot is then free at the barrier that publishes stage s + 1.  M = 600,
+// N = 8200, K = 1024: 47.2 -> 38.3 us (630 -> 787 TFLOP/s of f16 products).
 __device__ __forceinline__ f32x16 mfma_h(h8 a, h8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
-template <int NST>
+// Workgroup id -> (n tile, m tile): XCD x (id % 8) takes the x-th contiguous
+// range of the tiles numbered n-tile-major, so its L2 holds its own weight
+// columns and every XCD gets the same number of tiles whatever n_tiles is (65
+// at the head's 8200 columns: by whole n tiles one XCD would get 2 and seven 9).
+__device__ __forceinline__ bool f32_tile_of(int id, int n_tiles, int m_tiles, int& nt, int& mt) {
+  const int total = n_tiles * m_tiles, per = (total + 7) >> 3;
+  const int slot = id >> 3, p = (id & 7) * per + slot;
+  if (slot >= per || p >= total) return false;
+  nt = p / m_tiles;
+  mt = p - nt * m_tiles;
+  return true;
+}
+
+template <int BM, int NST>
 __global__ __launch_bounds__(256) void gemm_f32s_kernel(const GemmF32Args a) {
-  constexpr int STAGE = 16 * 1024;
+  constexpr int FM = BM / 64;                  // 32-row tiles of m per wavefront
+  constexpr int FRAGS = 8 + 2 * (BM / 32);     // per stage: (tile, plane)
+  constexpr int STAGE = FRAGS * 1024, OPS = FRAGS / 4;
   __shared__ __attribute__((aligned(16))) char smem[NST][STAGE];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wn = wave & 1, wm = wave >> 1;
-  const int n_tiles = (a.N + 127) / 128;
+  const int n_tiles = (a.N + 127) / 128, m_tiles = (a.M + BM - 1) / BM;
   int nt, mt;
-  if (!tile_of(blockIdx.x, n_tiles, nt, mt)) return;  // padding workgroup
+  if (!f32_tile_of(blockIdx.x, n_tiles, m_tiles, nt, mt)) return;  // padding workgroup
   const int64_t Ks = a.Ks;
   const int nst = (int)Ks;
-  // this wavefront's 4 fragments of every stage: waves 0-1 the weight
-  // fragments (4 column tiles x hi/lo), waves 2-3 the activation fragments
-  const _Float16* src[4];
+  // this wavefront's fragments of every stage: slots wave * OPS ..
+  const _Float16* src[OPS];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int idx = wave * 4 + t;  // fragment slot in the stage: (tile, plane)
-    const int tile = (idx & 7) >> 1, plane = idx & 1;
+  for (int t = 0; t < OPS; ++t) {
+    const int idx = wave * OPS + t, plane = idx & 1;
     if (idx < 8)
-      src[t] = (plane ? a.wlo : a.whi) + ((int64_t)(nt * 4 + tile) * Ks) * kFrag + lane * 8;
+      src[t] = (plane ? a.wlo : a.whi) + ((int64_t)(nt * 4 + (idx >> 1)) * Ks) * kFrag + lane * 8;
     else
-      src[t] = (plane ? a.alo : a.ahi) + ((int64_t)(mt * 4 + tile) * Ks) * kFrag + lane * 8;
+      src[t] = (plane ? a.alo : a.ahi) +
+               ((int64_t)(mt * (BM / 32) + ((idx - 8) >> 1)) * Ks) * kFrag + lane * 8;
   }
   auto issue = [&](int s) __attribute__((always_inline)) {
     char* base = smem[s % NST];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < OPS; ++t)
       __builtin_amdgcn_global_load_lds(static_cast<const void*>(src[t] + (int64_t)s * kFrag),
-                                       (lds_void_t*)(base + (wave * 4 + t) * 1024), 16, 0, 0);
+                                       (lds_void_t*)(base + (wave * OPS + t) * 1024), 16, 0, 0);
   };
-  f32x16 acc[2][2];
+  f32x16 acc[2][FM];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < FM; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
-#pragma unroll
-  for (int s = 0; s < NST - 1; ++s)
-    if (s < nst) issue(s);
-  for (int s = 0; s < nst; ++s) {
-    if (s + NST - 2 < nst)
-      wait_vm_lgkm<4 * (NST - 2)>();
-    else
-      wait_vm_lgkm<0>();
-    __builtin_amdgcn_s_barrier();
-    // the slot of stage s - 1, which every wavefront has read before the barrier
-    if (s + NST - 1 < nst) issue(s + NST - 1);
-    const char* base = smem[s % NST];
-    h8 wh[2], wl[2], ah[2], al[2];
+  h8 wh[2][2], wl[2][2], ah[2][FM], al[2][FM];  // [register set][tile]
+  auto read = [&](int s, int set) __attribute__((always_inline)) {
+    const char* base = smem[s % NST] + lane * 16;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      wh[i] = *reinterpret_cast<const h8*>(base + ((2 * wn + i) * 2 + 0) * 1024 + lane * 16);
-      wl[i] = *reinterpret_cast<const h8*>(base + ((2 * wn + i) * 2 + 1) * 1024 + lane * 16);
-      ah[i] = *reinterpret_cast<const h8*>(base + (8 + (2 * wm + i) * 2 + 0) * 1024 + lane * 16);
-      al[i] = *reinterpret_cast<const h8*>(base + (8 + (2 * wm + i) * 2 + 1) * 1024 + lane * 16);
+      wh[set][i] = *reinterpret_cast<const h8*>(base + ((2 * wn + i) * 2 + 0) * 1024);
+      wl[set][i] = *reinterpret_cast<const h8*>(base + ((2 * wn + i) * 2 + 1) * 1024);
     }
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+      ah[set][j] = *reinterpret_cast<const h8*>(base + (8 + (FM * wm + j) * 2 + 0) * 1024);
+      al[set][j] = *reinterpret_cast<const h8*>(base + (8 + (FM * wm + j) * 2 + 1) * 1024);
+    }
+  };
+  auto products = [&](auto par) __attribute__((always_inline)) {
+    constexpr int S = decltype(par)::value;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        acc[i][j] = mfma_h(wl[i], ah[j], acc[i][j]);
-        acc[i][j] = mfma_h(wh[i], al[j], acc[i][j]);
-        acc[i][j] = mfma_h(wh[i], ah[j], acc[i][j]);
+      for (int j = 0; j < FM; ++j) {
+        acc[i][j] = mfma_h(wl[S][i], ah[S][j], acc[i][j]);
+        acc[i][j] = mfma_h(wh[S][i], al[S][j], acc[i][j]);
+        acc[i][j] = mfma_h(wh[S][i], ah[S][j], acc[i][j]);
       }
+  };
+  // step s (not the last): stage s + 1 landed for every wavefront (up to NST - 2
+  // younger stages stay in flight), its fragments into the other set, then
+  // stage s's products.  No branch joins between the reads and the products:
+  // there the compiler would wait for the reads just issued.
+  auto step = [&](int s, auto par) __attribute__((always_inline)) {
+    constexpr int S = decltype(par)::value;
+    if (s + NST - 1 < nst)
+      wait_vm_lgkm<OPS * (NST - 2)>();
+    else
+      wait_vm_lgkm<0>();
+    wait_vm_lgkm<63>();  // (the compiler sees the reads done on every path)
+    __builtin_amdgcn_s_barrier();
+    if (s + NST < nst) issue(s + NST);  // stage s's slot: its fragments are in registers
+    read(s + 1, S ^ 1);
+    products(par);
+    // one read between two products: a wavefront's reads wait for their turn
+    // on the LDS port, all of them first would hold its products back
+#pragma unroll
+    for (int r = 0; r < 4 + 2 * FM; ++r) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 6 * FM, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+#pragma unroll
+  for (int s = 0; s < NST; ++s)
+    if (s < nst) issue(s);
+  if (NST - 1 < nst)
+    wait_vm_lgkm<OPS * (NST - 1)>();
+  else
+    wait_vm_lgkm<0>();
+  __builtin_amdgcn_s_barrier();
+  read(0, 0);
+  int s = 0;
+  for (; s + 2 < nst; s += 2) {
+    step(s, S0{});
+    step(s + 1, S1{});
+  }
+  if (s + 1 < nst) {
+    step(s, S0{});
+    products(S1{});
+  } else {
+    products(S0{});
   }
 
   // lane holds activation row m = tile + l % 32 and weight columns
   // n = tile + 8 (e / 4) + 4 (l / 32) + e % 4
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int64_t m = (int64_t)mt * 128 + wm * 64 + j * 32 + (lane & 31);
+  for (int j = 0; j < FM; ++j) {
+    const int64_t m = (int64_t)mt * BM + (wm * FM + j) * 32 + (lane & 31);
     if (m >= a.M) continue;
     const float sa = a.ascale[m];
     float* crow = a.C + m * a.ldc;
@@ -342,6 +458,16 @@ hipError_t launch_f32_weight(int64_t N, int64_t K, const float* src, int layout,
 
 hipError_t launch_f32_split(int64_t M, int64_t K, const float* A, int64_t Ks, _Float16* hi,
                             _Float16* lo, float* scale, hipStream_t st) {
+  if (K % 256 == 0 && K <= 1024 && ((uintptr_t)A & 15u) == 0) {
+    const dim3 grid((unsigned)((M + 3) / 4)), block(256);
+    switch (K / 256) {
+      case 1: hipLaunchKernelGGL(f32_split_rows_p_kernel<1>, grid, block, 0, st, M, A, hi, lo, scale); break;
+      case 2: hipLaunchKernelGGL(f32_split_rows_p_kernel<2>, grid, block, 0, st, M, A, hi, lo, scale); break;
+      case 3: hipLaunchKernelGGL(f32_split_rows_p_kernel<3>, grid, block, 0, st, M, A, hi, lo, scale); break;
+      default: hipLaunchKernelGGL(f32_split_rows_p_kernel<4>, grid, block, 0, st, M, A, hi, lo, scale); break;
+    }
+    return hipGetLastError();
+  }
   const int64_t Mp = (M + 127) / 128 * 128;
   hipLaunchKernelGGL(f32_split_rows_kernel, dim3((unsigned)Mp), dim3(256), 0, st, M, K, Ks, A, hi,
                      lo, scale);
@@ -365,10 +491,18 @@ hipError_t launch_rmsnorm_split(int64_t rows, int64_t cols, const float* x, cons
 
 hipError_t launch_gemm_f32(const GemmF32Args& a, hipStream_t st) {
   if (a.M <= 0 || a.N <= 0) return hipSuccess;
-  const int64_t n_tiles = (a.N + 127) / 128, m_tiles = (a.M + 127) / 128;
-  hipLaunchKernelGGL(gemm_f32s_kernel<4>, dim3((unsigned)grid_size(n_tiles, m_tiles)), dim3(256),
-                     0, st, a);
-  return hipGetLastError();
+  auto go = [&](auto kernel, int bm) {
+    const int64_t tiles = (((int64_t)a.N + 127) / 128) * (((int64_t)a.M + bm - 1) / bm);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(256), 0, st, a);
+    return hipGetLastError();
+  };
+  // 64-row tiles up to 1536 rows: more workgroups for few rows and a smaller
+  // last round (N = 8200, K = 1024, kernel us, 64 / 128 rows: M = 40 16.4 / 25.5,
+  // 300 26.0 / 29.3, 600 38.3 / 42.1, 1200 65.3 / 67.1); above, the 128-row
+  // tile's fewer LDS reads per product (M = 2000 whole call 131.7 / 125.6, 4000
+  // 240 / 232)
+  if (a.M <= 1536) return go(gemm_f32s_kernel<64, 4>, 64);
+  return go(gemm_f32s_kernel<128, 3>, 128);
 }
 
 }  // namespace ovh
