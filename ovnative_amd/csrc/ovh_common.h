@@ -64,6 +64,19 @@ __device__ __forceinline__ float group8_max(float v) {
   return v;
 }
 
+// Sum over the 8 lanes of an aligned 8-lane group, added left to right (lane 0
+// first), in every lane of the group (j = lane % 8).  Seven steps of "the lane
+// before's sum plus mine" (row_shr 1) leave lane 7 with ((s0 + s1) + ...) + s7;
+// then the upper quad takes it (quad_perm 3,3,3,3) and the lower one its mirror
+// (row_half_mirror).
+__device__ __forceinline__ float group8_sum_in_order(float s, int j) {
+  float t = s;
+#pragma unroll
+  for (int c = 0; c < 7; ++c) t = __fadd_rn(dpp_f32<0x111>(t), s);
+  const float up = dpp_f32<0xFF>(t), lo = dpp_f32<0x141>(up);
+  return j >= 4 ? up : lo;
+}
+
 // sum_{j<8} of lane j's p, added in lane order (every lane gets it); the lane
 // values are read as scalars (v_readlane), not through LDS.
 __device__ __forceinline__ float sum_lanes8_in_order(float p) {

@@ -36,7 +36,7 @@ __device__ __forceinline__ int64_t v_tile_index(int kvh, int64_t nkb, int64_t kb
 // group holds x[i] = element j + 8i, i = 0..15 (D = 128), i.e. the reference's
 // fma chain j, and both members of the rotation pairs (j + 8i, j + 8i + 64),
 // i < 8.  The chain runs in registers, the 8 chain sums are added left to right
-// after 7 lane reads; then xn = (x * scale) * w and the rotation
+// by lane moves; then xn = (x * scale) * w and the rotation
 // fmsub(na, c, nb s) / fmadd(na, s, nb c) with the row's cos/sin tables (TP:
 // a pointer to const float, in any address space).
 template <typename TP>
@@ -46,10 +46,7 @@ __device__ __forceinline__ void norm_rope_lanes8(float (&x)[16], const float* __
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < 16; ++i) s = fmaf(x[i], x[i], s);
-  const int g0 = (threadIdx.x & 63) & ~7;  // the group's first lane
-  float sum = __shfl(s, g0);
-#pragma unroll
-  for (int c = 1; c < 8; ++c) sum = __fadd_rn(sum, __shfl(s, g0 + c));
+  const float sum = group8_sum_in_order(s, j);
   const float scale = __fdiv_rn(1.f, sqrt_rn(__fadd_rn(__fdiv_rn(sum, (float)D), eps)));
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
