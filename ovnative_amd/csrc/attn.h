@@ -16,7 +16,7 @@ struct AttnSeg {
   int32_t rows;
   int64_t q_off;      // element offset into q and out
   int64_t kv_off;     // element offset into k and v
-  // Split-f16 kernel, mask form (launch_attention_split_only with mask_bits):
+  // Split-f16 kernel, mask form (launch_attention_split_only):
   // bit t % 32 of word [row * ((rows + 31) / 32) + t / 32] set = key t visible
   // (bias 0), clear = bias -1e30; nullptr = no mask.
   const uint32_t* bits;
@@ -67,7 +67,23 @@ struct AttnSplit {
   int64_t vt_cols;
   int64_t vt_off[kAttnMaxSegs];
   int32_t n_kv_heads;
-  uint32_t* overflow;  // set non-zero when a |k| or |v| is beyond the f16 range
+  // set non-zero when a |k| or |v| is beyond the f16 range (device memory, or, for
+  // launch_attention_split, pinned host memory)
+  uint32_t* overflow;
+  // launch_attention_split: the distinct biases of the segments, each turned into
+  // mask words (AttnSeg::bits points at them) as long as every value is 0 or
+  // -1e30; not_mask[m] = ticket (device memory, never `ticket` before the call)
+  // where one is not, and the segments of that bias are attended with its values.
+  // mask_of[s]: the bias of segment s, -1 without one.
+  uint64_t ticket;
+  uint64_t* not_mask;
+  int32_t n_masks;
+  struct {
+    const float* bias;
+    uint32_t* bits;
+    int32_t rows;
+  } masks[kAttnMaxSegs];
+  int8_t mask_of[kAttnMaxSegs];
   // Optional: the output quantised per 32-column block as s8_nk_quantize does
   // (codes [rows][out_stride], scales [rows][out_stride / 32]) instead of the
   // fp32 `out`; needs q_stride == out_stride and segment q offsets in whole rows.
@@ -81,10 +97,11 @@ struct AttnSplit {
 // Splits K and V of the segments into the planes, then attends.
 hipError_t launch_attention_split(const AttnArgs& args, const AttnSplit& sp, int max_rows,
                                   hipStream_t st);
-// Attention alone, over planes already written (launch_qk_norm_rope_split); the
-// segments' masks from AttnSeg::bits when mask_bits, else from AttnSeg::bias.
+// Attention alone, over planes already written; the segments' masks from
+// AttnSeg::bits, or (kMaskAuto) as launch_attention_split decides per bias.
+enum AttnMaskForm { kMaskBits, kMaskAuto };
 hipError_t launch_attention_split_only(const AttnArgs& args, const AttnSplit& sp, int max_rows,
-                                       bool mask_bits, hipStream_t st);
+                                       AttnMaskForm form, hipStream_t st);
 // launch_qk_norm_rope (D = 128) that also writes the planes of the roped k rows
 // of args' segments (args.kv_stride = n_kv_heads * 128) and of their V, in one
 // launch.

@@ -436,11 +436,42 @@ __device__ __forceinline__ bool split_v_job(const AttnArgs& a, const AttnSplit& 
   return split_v_tile(a, sp, s, kt, r >> 2, r & 3, tile, write_k);
 }
 
+// One row of a bias as mask bits, 64 keys per ballot: bit set = value 0 (key
+// visible), clear = -1e30; any other value in the row: true (no mask).
+__device__ __forceinline__ bool mask_row(const float* __restrict__ bias, int rows, int64_t row,
+                                         uint32_t* __restrict__ words, int lane) {
+  const int nw = (rows + 31) >> 5;
+  bool other = false;
+  for (int c = 0; c * 64 < rows; ++c) {
+    const int t = c * 64 + lane;
+    const float v = t < rows ? bias[row * rows + t] : -1e30f;
+    other |= !(v == 0.f || v == -1e30f);
+    const unsigned long long vis = __ballot(v == 0.f);
+    if (lane < 2 && 2 * c + lane < nw)
+      words[row * nw + 2 * c + lane] = (uint32_t)(vis >> (32 * lane));
+  }
+  return __any(other);
+}
+
 // Standalone split of K and V for one attention call: one workgroup per
-// (segment, key tile, KV head, dim quarter).
-__global__ __launch_bounds__(256) void split_kv_kernel(AttnArgs a, AttnSplit sp, int ktiles) {
+// (segment, key tile, KV head, dim quarter); then the masks' bit words, one
+// row per wavefront.
+__global__ __launch_bounds__(256) void split_kv_kernel(AttnArgs a, AttnSplit sp, int ktiles,
+                                                       int64_t kv_jobs) {
   __shared__ float tile[32][33];
-  if (split_v_job(a, sp, (int64_t)blockIdx.x, ktiles, tile, true)) atomicOr(sp.overflow, 1u);
+  if ((int64_t)blockIdx.x < kv_jobs) {
+    if (split_v_job(a, sp, (int64_t)blockIdx.x, ktiles, tile, true))
+      __hip_atomic_store(sp.overflow, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return;
+  }
+  int64_t j = (int64_t)blockIdx.x - kv_jobs;
+  int m = 0;
+  while (m + 1 < sp.n_masks && j >= (sp.masks[m].rows + 3) / 4) j -= (sp.masks[m++].rows + 3) / 4;
+  const int64_t row = 4 * j + (threadIdx.x >> 6);
+  if (row >= sp.masks[m].rows) return;
+  if (mask_row(sp.masks[m].bias, sp.masks[m].rows, row, sp.masks[m].bits, threadIdx.x & 63) &&
+      (threadIdx.x & 63) == 0)
+    __hip_atomic_store(sp.not_mask + m, sp.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The runner's form of qk-norm + RoPE + plane split, in one launch.  The first
@@ -541,16 +572,23 @@ constexpr float kMaskedLog2 = -1e29f * kLog2e;
 // The mask word of a segment without a mask: every key visible.
 __device__ const uint32_t kAllVisible[1] = {0xffffffffu};
 
+// The LDS of one workgroup of the short form.  The Q planes (2 x 32 x kQPad
+// halves) alias the start of `part`, which is written only after every wavefront
+// has left the key loop.  Rows of `part` are padded by 16 bytes, so that the
+// merge's reads (one query row per lane) spread over the banks.
+struct SplitLds {
+  float part[kAttnWaves][kAttnQ][kPartRow];
+  float mstat[kAttnWaves][kAttnQ], lstat[kAttnWaves][kAttnQ];
+  float alpha_s[kAttnWaves][kAttnQ];
+};
+
 template <bool kBits>
-__global__ __launch_bounds__(256, 2) void attention_split_kernel(AttnArgs args, AttnSplit sp,
-                                                                 int qtiles, int per_xcd) {
-  // The Q planes (2 x 32 x kQPad halves) alias the start of `part`, which is
-  // written only after every wavefront has left the key loop.  Rows of `part`
-  // are padded by 16 bytes, so that the merge's reads (one query row per lane)
-  // spread over the banks.
-  __shared__ __attribute__((aligned(16))) float part[kAttnWaves][kAttnQ][kPartRow];
-  __shared__ float mstat[kAttnWaves][kAttnQ], lstat[kAttnWaves][kAttnQ];
-  __shared__ float alpha_s[kAttnWaves][kAttnQ];
+__device__ __forceinline__ void attention_split_body(const AttnArgs& args, const AttnSplit& sp,
+                                                     int qtiles, int per_xcd, SplitLds& lds) {
+  auto& part = lds.part;
+  auto& mstat = lds.mstat;
+  auto& lstat = lds.lstat;
+  auto& alpha_s = lds.alpha_s;
   _Float16* qs_h = reinterpret_cast<_Float16*>(&part[0][0][0]);
   _Float16* qs_l = qs_h + kAttnQ * kQPad;
 
@@ -902,6 +940,35 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(AttnArgs args, 
 }
 
 
+template <bool kBits>
+__global__ __launch_bounds__(256, 2) void attention_split_kernel(AttnArgs args, AttnSplit sp,
+                                                                 int qtiles, int per_xcd) {
+  __shared__ __attribute__((aligned(16))) SplitLds lds;
+  attention_split_body<kBits>(args, sp, qtiles, per_xcd, lds);
+}
+
+// Whether segment s's bias must be read as values: it has one that the mask
+// pass of this call found to be no mask (uniform).
+__device__ __forceinline__ bool bias_values(const AttnSplit& sp, int s) {
+  const int m = sp.mask_of[s];
+  return m >= 0 && __builtin_amdgcn_readfirstlane((int)(sp.not_mask[m] == sp.ticket));
+}
+
+// The operator's form: a bias that is a mask (every value 0 or -1e30, as the
+// reference builds them) is attended through its bit words, 1/32 of the bytes
+// and with the K/V prefetch the float form has no registers for (2 x 300: 21.4
+// -> 15.2 us); any other through its values.  The same bits either way.
+__global__ __launch_bounds__(256, 2) void attention_split_auto_kernel(AttnArgs args, AttnSplit sp,
+                                                                      int qtiles, int per_xcd) {
+  __shared__ __attribute__((aligned(16))) SplitLds lds;
+  const int task = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+  if (task >= args.n_segs * args.n_heads * qtiles) return;
+  if (bias_values(sp, task / qtiles / args.n_heads))
+    attention_split_body<false>(args, sp, qtiles, per_xcd, lds);
+  else
+    attention_split_body<true>(args, sp, qtiles, per_xcd, lds);
+}
+
 // ---------------------------------------------------------------------------
 // Long-sequence form of the split-f16 attention.  In the form above every
 // workgroup (32 query rows) streams its KV head's whole planes through its
@@ -928,16 +995,12 @@ constexpr int kLdsMinTasks = 384;
 std::atomic<int64_t> g_long_min_tasks{kLdsMinTasks};
 
 template <bool kBits>
-__global__ __launch_bounds__(256, 2) void attention_split_lds_kernel(AttnArgs args, AttnSplit sp,
-                                                                     int qtiles, int per_xcd) {
-  // Double buffer as two arrays (kh, kl, vh, vl planes each): with the block
-  // loop unrolled by parity, a block's reads and the next block's DMA touch
-  // different arrays, which the compiler can tell apart (one array would make
-  // it wait for the DMA before every read).
-  __shared__ __attribute__((aligned(16))) _Float16 kv0[4][kLdsPlane];
-  __shared__ __attribute__((aligned(16))) _Float16 kv1[4][kLdsPlane];
-  __shared__ float xs[kAttnWaves][kAttnQ];                               // per-wave row exchange
-  __shared__ float ms[kAttnWaves][kAttnQ];
+__device__ __forceinline__ void attention_split_lds_body(const AttnArgs& args, const AttnSplit& sp,
+                                                         int qtiles, int per_xcd,
+                                                         _Float16 (&kv0)[4][kLdsPlane],
+                                                         _Float16 (&kv1)[4][kLdsPlane],
+                                                         float (&xs)[kAttnWaves][kAttnQ],
+                                                         float (&ms)[kAttnWaves][kAttnQ]) {
   const int G = args.group;  // 4 % G == 0 (host)
   // wave index in a scalar register: `live` and the block loop are uniform
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -982,7 +1045,8 @@ __global__ __launch_bounds__(256, 2) void attention_split_lds_kernel(AttnArgs ar
   // ---- DMA sources.  Wave w moves plane w of each block (8 x 1 KiB):
   // K planes (w < 2): slot s = 64 i + lane -> key s/16, chunk (s%16) ^ (key&15);
   // V planes: slot s -> row s/4, chunk (s%4) ^ ((row>>2)&3).
-  const _Float16* plane = (wave == 0 ? sp.kh : wave == 1 ? sp.kl : wave == 2 ? sp.vh : sp.vl) +
+  const _Float16 *const p0 = sp.kh, *const p1 = sp.kl, *const p2 = sp.vh, *const p3 = sp.vl;
+  const _Float16* plane = (wave == 0 ? p0 : wave == 1 ? p1 : wave == 2 ? p2 : p3) +
                           ((int64_t)kvh * (sp.vt_cols / 32) + sp.vt_off[sidx] / 32) * kTileHalves;
   auto issue = [&](int blk, auto odd) __attribute__((always_inline)) {
     const _Float16* pb = plane + (int64_t)blk * kTileHalves;  // the block's tiles
@@ -1196,14 +1260,46 @@ __global__ __launch_bounds__(256, 2) void attention_split_lds_kernel(AttnArgs ar
   }
 }
 
+// Double buffer as two arrays (kh, kl, vh, vl planes each): with the block
+// loop unrolled by parity, a block's reads and the next block's DMA touch
+// different arrays, which the compiler can tell apart (one array would make
+// it wait for the DMA before every read).
+#define OVH_ATTN_LONG_LDS                                              \
+  __shared__ __attribute__((aligned(16))) _Float16 kv0[4][kLdsPlane];  \
+  __shared__ __attribute__((aligned(16))) _Float16 kv1[4][kLdsPlane];  \
+  __shared__ float xs[kAttnWaves][kAttnQ]; /* per-wave row exchange */ \
+  __shared__ float ms[kAttnWaves][kAttnQ]
+
+template <bool kBits>
+__global__ __launch_bounds__(256, 2) void attention_split_lds_kernel(AttnArgs args, AttnSplit sp,
+                                                                     int qtiles, int per_xcd) {
+  OVH_ATTN_LONG_LDS;
+  attention_split_lds_body<kBits>(args, sp, qtiles, per_xcd, kv0, kv1, xs, ms);
+}
+
+// The operator's form, as attention_split_auto_kernel (16 x 1024, 8 masked: 531
+// -> 420 us; the float form reads each bias row once per head).
+__global__ __launch_bounds__(256, 2) void attention_split_lds_auto_kernel(AttnArgs args,
+                                                                          AttnSplit sp, int qtiles,
+                                                                          int per_xcd) {
+  OVH_ATTN_LONG_LDS;
+  const int n_kv = args.n_heads / args.group;
+  const int task = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+  if (task >= args.n_segs * n_kv * qtiles) return;
+  if (bias_values(sp, task / qtiles / n_kv))
+    attention_split_lds_body<false>(args, sp, qtiles, per_xcd, kv0, kv1, xs, ms);
+  else
+    attention_split_lds_body<true>(args, sp, qtiles, per_xcd, kv0, kv1, xs, ms);
+}
+#undef OVH_ATTN_LONG_LDS
+
 namespace {
 // resident workgroups per CU of the short form: a property of the kernel on
 // the architecture
-template <bool kBits>
 int split_occupancy() {
   static const int occ = [] {
     int o = 0;
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, attention_split_kernel<kBits>, 256, 0) ==
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, attention_split_kernel<true>, 256, 0) ==
                    hipSuccess
                ? o
                : 0;
@@ -1216,15 +1312,18 @@ hipError_t launch_attention_split(const AttnArgs& args, const AttnSplit& sp, int
                                   hipStream_t st) {
   if (args.n_segs <= 0 || max_rows <= 0) return hipSuccess;
   const int ktiles = (max_rows + 31) / 32;
-  const int64_t jobs = (int64_t)args.n_segs * ktiles * sp.n_kv_heads * 4;
-  hipLaunchKernelGGL(split_kv_kernel, dim3((unsigned)jobs), dim3(256), 0, st, args, sp, ktiles);
+  const int64_t kv_jobs = (int64_t)args.n_segs * ktiles * sp.n_kv_heads * 4;
+  int64_t jobs = kv_jobs;
+  for (int m = 0; m < sp.n_masks; ++m) jobs += (sp.masks[m].rows + 3) / 4;
+  hipLaunchKernelGGL(split_kv_kernel, dim3((unsigned)jobs), dim3(256), 0, st, args, sp, ktiles,
+                     kv_jobs);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  return launch_attention_split_only(args, sp, max_rows, false, st);
+  return launch_attention_split_only(args, sp, max_rows, kMaskAuto, st);
 }
 
 hipError_t launch_attention_split_only(const AttnArgs& args, const AttnSplit& sp, int max_rows,
-                                       bool mask_bits, hipStream_t st) {
+                                       AttnMaskForm form, hipStream_t st) {
   if (args.n_segs <= 0 || max_rows <= 0) return hipSuccess;
   if (sp.aq) {  // quantised output: whole rows of one stride, 32-column blocks
     if (args.q_stride != args.out_stride || args.out_stride % 32 != 0 || !sp.asc)
@@ -1249,12 +1348,9 @@ hipError_t launch_attention_split_only(const AttnArgs& args, const AttnSplit& sp
     const int tasks = lds_tasks;
     const int per_xcd = (tasks + 7) / 8;
     const dim3 grid((unsigned)(8 * per_xcd));
-    if (mask_bits)
-      hipLaunchKernelGGL(attention_split_lds_kernel<true>, grid, dim3(256), 0, st, args, sp, qtiles,
-                         per_xcd);
-    else
-      hipLaunchKernelGGL(attention_split_lds_kernel<false>, grid, dim3(256), 0, st, args, sp,
-                         qtiles, per_xcd);
+    auto kernel = form == kMaskBits ? attention_split_lds_kernel<true>
+                                    : attention_split_lds_auto_kernel;
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, args, sp, qtiles, per_xcd);
     return hipGetLastError();
   }
   // 1-D grid of 8 * per_xcd workgroups (XCD-aware task order in the kernel),
@@ -1264,11 +1360,12 @@ hipError_t launch_attention_split_only(const AttnArgs& args, const AttnSplit& sp
   const int per_xcd = (tasks + 7) / 8;
   // the prefetch workgroups only where all of them are resident beside the
   // attention's own (else they would run after them and lengthen the launch)
-  auto kernel = mask_bits ? attention_split_kernel<true> : attention_split_kernel<false>;
+  auto kernel = form == kMaskBits ? attention_split_kernel<true> : attention_split_auto_kernel;
   AttnSplit s = sp;
   if (!s.pf.p || s.pf.bytes <= 0 || s.pf.wgs <= 0 ||
       8 * (int64_t)(per_xcd + s.pf.wgs) >
-          (int64_t)(mask_bits ? split_occupancy<true>() : split_occupancy<false>()) * device_cus())
+          (int64_t)split_occupancy() * device_cus() ||
+      form != kMaskBits)
     s.pf.wgs = 0;
   const dim3 grid((unsigned)(8 * per_xcd + 8 * s.pf.wgs));
   hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, args, s, qtiles, per_xcd);

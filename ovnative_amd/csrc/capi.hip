@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <condition_variable>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -306,6 +307,112 @@ int linear_q_sliced(int64_t M, const int8_t* aq, const float* asc, const OvhWeig
 }
 }  // namespace ovh
 
+namespace {
+constexpr int kMaxDevices = 64;
+
+// A call's workspace, stream-ordered (hipFreeAsync after the last launch): from
+// a pool of the library's own per device, which keeps up to kPoolKeep bytes
+// between calls and gives the rest back at the next synchronisation.  The
+// device's default pool keeps nothing, so that every synchronising call pays
+// for mapping and unmapping its workspace.  Each call owns its allocation: any
+// number of threads and streams.  A call under graph capture allocates in the
+// graph, from the default pool.
+constexpr uint64_t kPoolKeep = (uint64_t)256 << 20;
+std::mutex g_pool_mu;
+hipMemPool_t g_pool[kMaxDevices] = {};
+bool g_pool_tried[kMaxDevices] = {};
+
+hipMemPool_t call_pool(int dev) {
+  if (dev < 0 || dev >= kMaxDevices) return nullptr;
+  std::lock_guard<std::mutex> lock(g_pool_mu);
+  if (!g_pool_tried[dev]) {
+    g_pool_tried[dev] = true;
+    hipMemPoolProps props{};
+    props.allocType = hipMemAllocationTypePinned;
+    props.handleTypes = hipMemHandleTypeNone;
+    props.location.type = hipMemLocationTypeDevice;
+    props.location.id = dev;
+    hipMemPool_t p = nullptr;
+    uint64_t keep = kPoolKeep;
+    if (hipMemPoolCreate(&p, &props) != hipSuccess) {
+      (void)hipGetLastError();
+    } else if (hipMemPoolSetAttribute(p, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
+      (void)hipGetLastError();
+      (void)hipMemPoolDestroy(p);
+    } else {
+      g_pool[dev] = p;
+    }
+  }
+  return g_pool[dev];
+}
+
+hipError_t call_malloc(void** ptr, size_t bytes, hipStream_t st) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  hipError_t e = hipStreamIsCapturing(st, &cap);
+  if (e != hipSuccess) return e;
+  int dev = -1;
+  if (cap == hipStreamCaptureStatusNone && hipGetDevice(&dev) == hipSuccess)
+    if (hipMemPool_t pool = call_pool(dev)) return hipMallocFromPoolAsync(ptr, bytes, pool, st);
+  return hipMallocAsync(ptr, bytes, st);
+}
+
+// What a split-attention call reports while it runs: a pinned host word (|k| or
+// |v| beyond f16) and device words for its biases, one slot per call in flight.
+// The device words compare with the call's ticket, so nothing is cleared between
+// calls (a launch of its own); tickets never repeat.
+constexpr int kAttnSlots = 32;
+__device__ uint64_t attn_not_mask[kAttnSlots][ovh::kAttnMaxSegs];
+struct AttnSlots {
+  std::mutex mu;
+  std::condition_variable freed;
+  uint32_t busy = 0;               // bit per slot
+  uint32_t* overflow = nullptr;    // pinned, [kAttnSlots], one word per 64 bytes
+  uint64_t* not_mask[kMaxDevices] = {};
+  uint64_t ticket = 0;
+};
+AttnSlots g_attn;
+
+struct AttnSlot {
+  int i = -1;
+  volatile uint32_t* overflow = nullptr;
+  uint64_t* not_mask = nullptr;
+  uint64_t ticket = 0;
+  hipError_t take() {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
+    std::unique_lock<std::mutex> lock(g_attn.mu);
+    if (!g_attn.overflow) {
+      void* p = nullptr;
+      e = hipHostMalloc(&p, 64 * kAttnSlots, hipHostMallocPortable);
+      if (e != hipSuccess) return e;
+      g_attn.overflow = static_cast<uint32_t*>(p);
+    }
+    if (!g_attn.not_mask[dev]) {
+      void* p = nullptr;
+      e = hipGetSymbolAddress(&p, HIP_SYMBOL(attn_not_mask));
+      if (e != hipSuccess) return e;
+      g_attn.not_mask[dev] = static_cast<uint64_t*>(p);
+    }
+    g_attn.freed.wait(lock, [] { return g_attn.busy != ~0u; });
+    i = __builtin_ctz(~g_attn.busy);
+    g_attn.busy |= 1u << i;
+    overflow = g_attn.overflow + 16 * i;
+    *overflow = 0;
+    not_mask = g_attn.not_mask[dev] + i * ovh::kAttnMaxSegs;
+    ticket = ++g_attn.ticket;
+    return hipSuccess;
+  }
+  ~AttnSlot() {
+    if (i < 0) return;
+    std::lock_guard<std::mutex> lock(g_attn.mu);
+    g_attn.busy &= ~(1u << i);
+    g_attn.freed.notify_one();
+  }
+};
+}  // namespace
+
 extern "C" {
 
 const char* ovh_last_error(void) { return t_err.c_str(); }
@@ -461,8 +568,8 @@ int ovh_linear_f32(int64_t M, const float* A, const OvhWeight* w, float* C, int6
   const size_t plane = sizeof(_Float16) * (size_t)ovh::f32_plane_halves(M, fw.K);
   const size_t rows = (size_t)((M + 127) / 128 * 128);
   char* ws = nullptr;
-  OVH_HIP(hipMallocAsync(reinterpret_cast<void**>(&ws), 2 * plane + sizeof(float) * rows, st),
-          "hipMallocAsync(linear_f32)");
+  OVH_HIP(call_malloc(reinterpret_cast<void**>(&ws), 2 * plane + sizeof(float) * rows, st),
+          "workspace of linear_f32");
   ovh::GemmF32Args a;
   a.M = (int)M;
   a.N = (int)fw.N;
@@ -758,7 +865,6 @@ int ovh_diag_read(const void* src, int64_t bytes, int path, void* stream) {
 namespace {
 constexpr size_t kNoAllocScratchBytes = (size_t)16 << 20;
 static __device__ __align__(256) int8_t scratch[kNoAllocScratchBytes];
-constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 void* g_scratch[kMaxDevices] = {};
 
@@ -978,24 +1084,49 @@ int ovh_attention_split(const OvhAttnSegment* segs, int n_segs, int n_heads, int
     max_rows = g.rows > max_rows ? g.rows : max_rows;
   }
   sp.n_kv_heads = n_kv_heads;
+  // the distinct biases, for their mask words
+  size_t mask_words = 0;
+  size_t mask_at[ovh::kAttnMaxSegs];
+  for (int s = 0; s < n_segs; ++s) {
+    const OvhAttnSegment& g = segs[s];
+    sp.mask_of[s] = -1;
+    if (!g.bias || g.rows <= 0) continue;
+    int m = 0;
+    while (m < sp.n_masks && (sp.masks[m].bias != g.bias || sp.masks[m].rows != g.rows)) ++m;
+    if (m == sp.n_masks) {
+      sp.masks[m].bias = g.bias;
+      sp.masks[m].rows = g.rows;
+      mask_at[m] = mask_words;
+      mask_words += (size_t)g.rows * (size_t)((g.rows + 31) / 32);
+      ++sp.n_masks;
+    }
+    sp.mask_of[s] = (int8_t)m;
+  }
   hipStream_t st = as_stream(stream);
   const size_t vbytes = sizeof(_Float16) * (size_t)((int64_t)n_kv_heads * head_dim * sp.vt_cols);
   const size_t kbytes = vbytes;  // K and V planes are both tile-major over the padded keys
   char* ws = nullptr;
-  const size_t total = 2 * kbytes + 2 * vbytes + 256;
-  OVH_HIP(hipMallocAsync(reinterpret_cast<void**>(&ws), total, st), "hipMallocAsync(split)");
+  const size_t total = 2 * kbytes + 2 * vbytes + sizeof(uint32_t) * mask_words + 256;
+  AttnSlot slot;
+  OVH_HIP(slot.take(), "attention_split report slot");
+  OVH_HIP(call_malloc(reinterpret_cast<void**>(&ws), total, st), "workspace of attention_split");
   sp.kh = reinterpret_cast<_Float16*>(ws);
   sp.kl = reinterpret_cast<_Float16*>(ws + kbytes);
   sp.vh = reinterpret_cast<_Float16*>(ws + 2 * kbytes);
   sp.vl = reinterpret_cast<_Float16*>(ws + 2 * kbytes + vbytes);
-  sp.overflow = reinterpret_cast<uint32_t*>(ws + 2 * kbytes + 2 * vbytes);
-  hipError_t e = hipMemsetAsync(sp.overflow, 0, sizeof(uint32_t), st);
-  if (e == hipSuccess) e = ovh::launch_attention_split(a, sp, max_rows, st);
-  uint32_t flag = 0;
-  if (e == hipSuccess) e = hipMemcpyAsync(&flag, sp.overflow, sizeof flag, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  uint32_t* const words = reinterpret_cast<uint32_t*>(ws + 2 * kbytes + 2 * vbytes);
+  for (int m = 0; m < sp.n_masks; ++m) sp.masks[m].bits = words + mask_at[m];
+  for (int s = 0; s < n_segs; ++s)
+    if (sp.mask_of[s] >= 0) a.segs[s].bits = sp.masks[sp.mask_of[s]].bits;
+  sp.overflow = const_cast<uint32_t*>(slot.overflow);
+  sp.ticket = slot.ticket;
+  sp.not_mask = slot.not_mask;
+  hipError_t e = ovh::launch_attention_split(a, sp, max_rows, st);
   (void)hipFreeAsync(ws, st);
+  const hipError_t es = hipStreamSynchronize(st);
+  if (e == hipSuccess) e = es;
   if (e != hipSuccess) return hip_fail(e, "attention_split");
+  const uint32_t flag = *slot.overflow;
   if (flag)
     return fail(OV_ERR_INVALID_ARG, "attention_split: |k| or |v| beyond the f16 range; use "
                                     "ovh_attention");

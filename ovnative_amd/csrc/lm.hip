@@ -1059,7 +1059,7 @@ int forward_rows(OvhLm& L, int batch, int seq, const std::vector<SegIn>& segs,
         OVH_HIP(ovh::launch_gemm(ga, ovh::kQkvNorm, st), "q/k/v + qk-norm launch");
         if ((rc = mark("qkv")) != OV_OK) return rc;
         sp.pf = prefetch_of(Y.o, kPfAttnWgs);
-        OVH_HIP(ovh::launch_attention_split_only(aargs, sp, max_rows, true, st), "attention launch");
+        OVH_HIP(ovh::launch_attention_split_only(aargs, sp, max_rows, ovh::kMaskBits, st), "attention launch");
         sp.pf = ovh::L2Prefetch{};
       } else if ((rc = ovh::linear_q_sliced(T, aq, asc, Y.qkv, qkv_n, qkv_c, 3, st, tiled, aq16,
                                             f16)) != OV_OK || (rc = mark("qkv")) != OV_OK) {
@@ -1070,7 +1070,7 @@ int forward_rows(OvhLm& L, int batch, int seq, const std::vector<SegIn>& segs,
                                                sinb, c.rms_eps, aargs, sp, max_rows, st),
                 "qk_norm_rope launch");
         if ((rc = mark("qk_norm_rope")) != OV_OK) return rc;
-        OVH_HIP(ovh::launch_attention_split_only(aargs, sp, max_rows, true, st), "attention launch");
+        OVH_HIP(ovh::launch_attention_split_only(aargs, sp, max_rows, ovh::kMaskBits, st), "attention launch");
       } else {
         if ((rc = ovh_qk_norm_rope(q, k, Y.qn, Y.kn, T, c.n_heads, c.n_kv_heads, (int)D, cosb,
                                    sinb, c.rms_eps, st)) != OV_OK ||
