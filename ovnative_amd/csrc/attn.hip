@@ -436,35 +436,43 @@ __device__ __forceinline__ bool split_v_job(const AttnArgs& a, const AttnSplit& 
   return split_v_tile(a, sp, s, kt, r >> 2, r & 3, tile, write_k);
 }
 
-// One row of a bias as mask bits, 64 keys per ballot: bit set = value 0 (key
-// visible), clear = -1e30; any other value in the row: true (no mask).
+// One row of a bias as mask bits, 64 keys per ballot, four ballots' loads in
+// flight: bit set = value 0 (key visible), clear = -1e30; any other value in the
+// row: true (no mask).
 __device__ __forceinline__ bool mask_row(const float* __restrict__ bias, int rows, int64_t row,
                                          uint32_t* __restrict__ words, int lane) {
   const int nw = (rows + 31) >> 5;
   bool other = false;
-  for (int c = 0; c * 64 < rows; ++c) {
-    const int t = c * 64 + lane;
-    const float v = t < rows ? bias[row * rows + t] : -1e30f;
-    other |= !(v == 0.f || v == -1e30f);
-    const unsigned long long vis = __ballot(v == 0.f);
-    if (lane < 2 && 2 * c + lane < nw)
-      words[row * nw + 2 * c + lane] = (uint32_t)(vis >> (32 * lane));
+  for (int c0 = 0; c0 * 64 < rows; c0 += 4) {
+    float v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int t = (c0 + u) * 64 + lane;
+      v[u] = t < rows ? bias[row * rows + t] : -1e30f;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      other |= !(v[u] == 0.f || v[u] == -1e30f);
+      const unsigned long long vis = __ballot(v[u] == 0.f);
+      const int w = 2 * (c0 + u) + lane;
+      if (lane < 2 && w < nw) words[row * nw + w] = (uint32_t)(vis >> (32 * lane));
+    }
   }
   return __any(other);
 }
 
-// Standalone split of K and V for one attention call: one workgroup per
-// (segment, key tile, KV head, dim quarter); then the masks' bit words, one
-// row per wavefront.
+// Standalone split of K and V for one attention call: first the masks' bit
+// words, one row per wavefront (a row is a chain of loads, so these start with
+// the launch), then one workgroup per (segment, key tile, KV head, dim quarter).
 __global__ __launch_bounds__(256) void split_kv_kernel(AttnArgs a, AttnSplit sp, int ktiles,
-                                                       int64_t kv_jobs) {
+                                                       int64_t mask_jobs) {
   __shared__ float tile[32][33];
-  if ((int64_t)blockIdx.x < kv_jobs) {
-    if (split_v_job(a, sp, (int64_t)blockIdx.x, ktiles, tile, true))
+  int64_t j = blockIdx.x;
+  if (j >= mask_jobs) {
+    if (split_v_job(a, sp, j - mask_jobs, ktiles, tile, true))
       __hip_atomic_store(sp.overflow, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     return;
   }
-  int64_t j = (int64_t)blockIdx.x - kv_jobs;
   int m = 0;
   while (m + 1 < sp.n_masks && j >= (sp.masks[m].rows + 3) / 4) j -= (sp.masks[m++].rows + 3) / 4;
   const int64_t row = 4 * j + (threadIdx.x >> 6);
@@ -1313,10 +1321,10 @@ hipError_t launch_attention_split(const AttnArgs& args, const AttnSplit& sp, int
   if (args.n_segs <= 0 || max_rows <= 0) return hipSuccess;
   const int ktiles = (max_rows + 31) / 32;
   const int64_t kv_jobs = (int64_t)args.n_segs * ktiles * sp.n_kv_heads * 4;
-  int64_t jobs = kv_jobs;
-  for (int m = 0; m < sp.n_masks; ++m) jobs += (sp.masks[m].rows + 3) / 4;
-  hipLaunchKernelGGL(split_kv_kernel, dim3((unsigned)jobs), dim3(256), 0, st, args, sp, ktiles,
-                     kv_jobs);
+  int64_t mask_jobs = 0;
+  for (int m = 0; m < sp.n_masks; ++m) mask_jobs += (sp.masks[m].rows + 3) / 4;
+  hipLaunchKernelGGL(split_kv_kernel, dim3((unsigned)(mask_jobs + kv_jobs)), dim3(256), 0, st, args,
+                     sp, ktiles, mask_jobs);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   return launch_attention_split_only(args, sp, max_rows, kMaskAuto, st);
