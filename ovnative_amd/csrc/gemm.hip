@@ -385,7 +385,9 @@ __device__ __forceinline__ bool qkv_tile_of(int id, int q_tiles, int n_tiles, in
 // tiles moved as two 1 KiB DMA units, 16-byte fragments, fp32 block products.
 // The body of one workgroup's output tile; wg is the workgroup's index in its
 // GEMM's grid (grouped launches offset it).
-template <int BN, int BM, int WN, int WM, int SB, int NST, int MODE, bool PIPE, bool F16 = false>
+// TMAJ: codes tile-major, else row-major (in LDS by rows, or in the row-chunk
+// order; below).
+template <int BN, int BM, int WN, int WM, int SB, int NST, int MODE, bool PIPE, bool F16, bool TMAJ>
 __device__ __forceinline__ void gemm16_tile(const GemmArgs& a, const int wg) {
   constexpr int NW = WN * WM;
   constexpr int TN = BN / WN, TM = BM / WM;
@@ -396,6 +398,7 @@ __device__ __forceinline__ void gemm16_tile(const GemmArgs& a, const int wg) {
   static_assert((SB % 4 == 0 || SB == 2) && NST >= 2,
                 "scales move in 16-byte (4-block) chunks, or per block for 2-block stages");
   static_assert(!F16 || MODE != kDumpBlocks, "block dumps on the int8 operands only");
+  static_assert(TMAJ || (!F16 && SB >= 4), "row-major codes: int8, whole 128-byte lines of a row");
   constexpr int WT = BN / 32, AT = BM / 32;
   constexpr int U = F16 ? 2 : 1;          // 1 KiB DMA units per block tile
   constexpr int TB = TILE * U;            // bytes per block tile
@@ -449,6 +452,20 @@ __device__ __forceinline__ void gemm16_tile(const GemmArgs& a, const int wg) {
   // wavefront w takes idx = w, w + NW, ...
   const int8_t* const wsrc = F16 ? reinterpret_cast<const int8_t*>(a.W16) : a.W;
   const int8_t* const asrc = F16 ? reinterpret_cast<const int8_t*>(a.aq16) : a.aq;
+  // Row-major codes.  By rows: unit bb of a 32-row tile is 32 / SB whole rows of
+  // the stage, 32 SB contiguous bytes each, so an op touches 8 lines; slot i of
+  // row rr in LDS holds the row's bytes 16 (i ^ row_swz(rr)) .., so that a
+  // fragment read's 16 rows fall on different banks.  Row-chunk: unit bb is block
+  // bb of the 32 rows (32 lines an op), and the fragment reads need no permuted
+  // address (a VALU instruction each).  The pipelined tiles, which wait for the
+  // DMA, take the rows (N = 1024, M = 600: K = 2048 11.6 -> 9.6 us, 3072 15.6 ->
+  // 12.2; M = 1536, K = 3072 31.3 -> 24.5); the large-M tile, bound by VALU issue,
+  // the chunks (M = 2048, K = 2048 20.3 against 22.3).
+  constexpr bool ROWS = !TMAJ && PIPE;
+  constexpr int kSlotsRow = 2 * SB;
+  auto row_swz = [](int rr) __attribute__((always_inline)) {
+    return (rr * SB / 8) % kSlotsRow;
+  };
   const int8_t* src[TPW];
   int64_t step[TPW];
 #pragma unroll
@@ -460,13 +477,15 @@ __device__ __forceinline__ void gemm16_tile(const GemmArgs& a, const int wg) {
     if (r < WT) {
       src[t] = wsrc + ((int64_t)(n0 / 32 + r) * Kb + bb) * TB + h * TILE + lane * 16;
       step[t] = (int64_t)SB * TB;
-    } else if (F16 || a.a_tiled) {
+    } else if constexpr (TMAJ) {
       src[t] = asrc + ((int64_t)(m0 / 32 + r - WT) * Kb + bb) * TB + h * TILE + lane * 16;
       step[t] = (int64_t)SB * TB;
     } else {
-      int row = m0 + (r - WT) * 32 + (lane & 31);
+      const int rr = ROWS ? bb * (32 / SB) + lane / kSlotsRow : lane & 31;
+      int row = m0 + (r - WT) * 32 + rr;
       row = row < a.M ? row : a.M - 1;  // rows are independent: clamp, discard later
-      src[t] = a.aq + (int64_t)row * Kp + bb * 32 + (lane >> 5) * 16;
+      src[t] = a.aq + (int64_t)row * Kp +
+               (ROWS ? ((lane % kSlotsRow) ^ row_swz(rr)) * 16 : bb * 32 + (lane >> 5) * 16);
       step[t] = SB * 32;
     }
   }
@@ -517,9 +536,8 @@ __device__ __forceinline__ void gemm16_tile(const GemmArgs& a, const int wg) {
   const bool last_wave = wave == NW - 1, hi_wave = EVEN || wave < TILES % NW;
   // fragment byte offsets inside a block tile (see above): weights and
   // tile-major codes in the interleaved layout, lane l's 8 bytes at 512 h + 8 l
-  // (linear); row-major codes as the DMA gathered them, row-chunk order
+  // (linear); row-major codes: byte 32 bb + 8 (l / 16) of the row, permuted
   const int q = lane >> 4;
-  const int frag_rows = ((q >> 1) * 32 + (lane & 15)) * 16 + (q & 1) * 8;
   int aoff[FN], boff[FM];
 #pragma unroll
   for (int i = 0; i < FN; ++i) {
@@ -529,10 +547,18 @@ __device__ __forceinline__ void gemm16_tile(const GemmArgs& a, const int wg) {
 #pragma unroll
   for (int j = 0; j < FM; ++j) {
     const int t16 = wm * FM + j;
+    const int rr = (t16 & 1) * 16 + (lane & 15);
     boff[j] = (WT + (t16 >> 1)) * SB * TB +
-              ((F16 || a.a_tiled) ? (t16 & 1) * (TB / 2) + FB * lane
-                                  : (t16 & 1) * 16 * 16 + frag_rows);
+              (TMAJ   ? (t16 & 1) * (TB / 2) + FB * lane
+               : ROWS ? rr * SB * 32 + ((q >> 1) ^ (row_swz(rr) & 1)) * 16 + (q & 1) * 8
+                      : ((q >> 1) * 32 + rr) * 16 + (q & 1) * 8);
   }
+  // (the two 16-row halves of a tile have the same permutation)
+  const int bxor = !ROWS ? 0 : (row_swz(lane & 15) & ~1) * 16;
+  static_assert(!ROWS || 16 * SB / 8 % kSlotsRow == 0, "rows rr and rr + 16 permuted alike");
+  auto read_b = [&](const int8_t* base, int j, int bb) __attribute__((always_inline)) {
+    return *reinterpret_cast<const Frag*>(base + boff[j] + (!ROWS ? bb * TB : (bb * 32) ^ bxor));
+  };
 
   f32x4 f[FN][FM];
 #pragma unroll
@@ -591,7 +617,7 @@ __device__ __forceinline__ void gemm16_tile(const GemmArgs& a, const int wg) {
         af[bb][i] = *reinterpret_cast<const Frag*>(base + aoff[i] + bb * TB);
 #pragma unroll
       for (int j = 0; j < FM; ++j)
-        bf[bb][j] = *reinterpret_cast<const Frag*>(base + boff[j] + bb * TB);
+        bf[bb][j] = read_b(base, j, bb);
     }
   };
   auto products = [&]() __attribute__((always_inline)) {
@@ -689,7 +715,7 @@ __device__ __forceinline__ void gemm16_tile(const GemmArgs& a, const int wg) {
           a1[i] = *reinterpret_cast<const Frag*>(base + aoff[i] + bb * TB);
 #pragma unroll
         for (int j = 0; j < FM; ++j)
-          b1[j] = *reinterpret_cast<const Frag*>(base + boff[j] + bb * TB);
+          b1[j] = read_b(base, j, bb);
 #pragma unroll
         for (int i = 0; i < FN; ++i)
 #pragma unroll
@@ -1074,9 +1100,10 @@ __device__ __forceinline__ void gemm16_tile(const GemmArgs& a, const int wg) {
   }
 }
 
-template <int BN, int BM, int WN, int WM, int SB, int NST, int MODE, bool PIPE, bool F16 = false>
+template <int BN, int BM, int WN, int WM, int SB, int NST, int MODE, bool PIPE, bool F16 = false,
+          bool TMAJ = true>
 __global__ __launch_bounds__(64 * WN * WM) void gemm16_kernel(const GemmArgs a) {
-  gemm16_tile<BN, BM, WN, WM, SB, NST, MODE, PIPE, F16>(a, blockIdx.x);
+  gemm16_tile<BN, BM, WN, WM, SB, NST, MODE, PIPE, F16, TMAJ>(a, blockIdx.x);
 }
 
 // Several independent GEMMs in one launch: GEMM g takes the workgroups
@@ -1086,7 +1113,8 @@ template <int BN, int BM, int WN, int WM, int SB, int NST, int MODE, bool PIPE>
 __global__ __launch_bounds__(64 * WN * WM) void gemm16_grouped_kernel(const GemmGroups gg) {
   int g = 0;
   while (g + 1 < gg.n && (int)blockIdx.x >= gg.start[g + 1]) ++g;
-  gemm16_tile<BN, BM, WN, WM, SB, NST, MODE, PIPE>(gg.args[g], (int)blockIdx.x - gg.start[g]);
+  gemm16_tile<BN, BM, WN, WM, SB, NST, MODE, PIPE, false, false>(gg.args[g],
+                                                                 (int)blockIdx.x - gg.start[g]);
 }
 
 // Launchable when Kb % SB == 0.
@@ -1095,15 +1123,20 @@ hipError_t launch_cfg16(const GemmArgs& a, GemmMode mode, hipStream_t st) {
   if (a.Kb % SB) return hipErrorInvalidValue;
   const int64_t n_tiles = ((int64_t)a.N + BN - 1) / BN, m_tiles = ((int64_t)a.M + BM - 1) / BM;
   const dim3 grid((unsigned)grid_size(n_tiles, m_tiles)), block(64 * WN * WM);
-  if (mode == kAccumulate)
-    hipLaunchKernelGGL((gemm16_kernel<BN, BM, WN, WM, SB, NST, kAccumulate, PIPE>), grid, block, 0,
-                       st, a);
-  else if (mode == kDumpBlocks)
-    hipLaunchKernelGGL((gemm16_kernel<BN, BM, WN, WM, SB, NST, kDumpBlocks, PIPE>), grid, block, 0,
-                       st, a);
-  else
-    hipLaunchKernelGGL((gemm16_kernel<BN, BM, WN, WM, SB, NST, kStore, PIPE>), grid, block, 0, st, a);
-  return hipGetLastError();
+  auto go = [&](auto tiled) {
+    constexpr bool TMAJ = decltype(tiled)::value;
+    if (mode == kAccumulate)
+      hipLaunchKernelGGL((gemm16_kernel<BN, BM, WN, WM, SB, NST, kAccumulate, PIPE, false, TMAJ>),
+                         grid, block, 0, st, a);
+    else if (mode == kDumpBlocks)
+      hipLaunchKernelGGL((gemm16_kernel<BN, BM, WN, WM, SB, NST, kDumpBlocks, PIPE, false, TMAJ>),
+                         grid, block, 0, st, a);
+    else
+      hipLaunchKernelGGL((gemm16_kernel<BN, BM, WN, WM, SB, NST, kStore, PIPE, false, TMAJ>), grid,
+                         block, 0, st, a);
+    return hipGetLastError();
+  };
+  return a.a_tiled ? go(std::true_type{}) : go(std::false_type{});
 }
 
 // The SiLU-fused mode (wave tiles 64 rows wide: BN / WN == 64).
@@ -1113,8 +1146,12 @@ hipError_t launch_cfg16_silu(const GemmArgs& a, hipStream_t st) {
   if (a.Kb % SB || a.N % 128 || !a.hq || !a.hsc || a.hKp < a.N / 2) return hipErrorInvalidValue;
   const int64_t n_tiles = ((int64_t)a.N + BN - 1) / BN, m_tiles = ((int64_t)a.M + BM - 1) / BM;
   const dim3 grid((unsigned)grid_size(n_tiles, m_tiles)), block(64 * WN * WM);
-  hipLaunchKernelGGL((gemm16_kernel<BN, BM, WN, WM, SB, NST, kSiluQuant, PIPE>), grid, block, 0, st,
-                     a);
+  if (a.a_tiled)
+    hipLaunchKernelGGL((gemm16_kernel<BN, BM, WN, WM, SB, NST, kSiluQuant, PIPE, false, true>), grid,
+                       block, 0, st, a);
+  else
+    hipLaunchKernelGGL((gemm16_kernel<BN, BM, WN, WM, SB, NST, kSiluQuant, PIPE, false, false>),
+                       grid, block, 0, st, a);
   return hipGetLastError();
 }
 
@@ -1170,7 +1207,8 @@ hipError_t launch_qkv_cfg(const GemmArgs& a, hipStream_t st) {
 }
 
 hipError_t launch_qkv_norm(const GemmArgs& a, hipStream_t st) {
-  if (a.Kb % 4 || !a.qf || !a.qnw || !a.knw || a.N % 128) return hipErrorInvalidValue;
+  if (a.Kb % 4 || !a.a_tiled || !a.qf || !a.qnw || !a.knw || a.N % 128)
+    return hipErrorInvalidValue;
   if (a.W16 && a.aq16) return launch_qkv_cfg<32, true, true>(a, st);
   if (a.M >= 2048) return launch_qkv_cfg<64, false, false>(a, st);
   return launch_qkv_cfg<32, true, false>(a, st);
@@ -1249,7 +1287,7 @@ hipError_t launch_norm_cfg(const GemmArgs& a, int64_t slot0, hipStream_t st) {
 // rows slots kLargeMBandBase on; each class has one column-tile count per N,
 // which is what a slot's counter advances by per launch.
 hipError_t launch_gemm_norm(const GemmArgs& a, hipStream_t st) {
-  if (a.Kb % 4 || a.nslices != 1 || !a.out[0] || !a.nw || !a.nq || !a.nsc || !a.band_cnt ||
+  if (a.Kb % 4 || !a.a_tiled || a.nslices != 1 || !a.out[0] || !a.nw || !a.nq || !a.nsc || !a.band_cnt ||
       !a.norm_err || a.N % 256 || a.N < 256 || a.N > 1024 || a.W16 || a.aq16)
     return hipErrorInvalidValue;
   // the band placement takes workgroup id % 8 for the XCD
