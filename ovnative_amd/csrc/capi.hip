@@ -785,6 +785,16 @@ int linear_workspace(hipStream_t st, size_t bytes, void** ptr, bool* owned) {
   *ptr = ws->ptr;
   return OV_OK;
 }
+
+// The arguments are ones ovh::linear_q takes, the int8 form is asked for, and
+// the one-launch form is the faster one; anything else, errors included, goes
+// the general way.
+bool linear_one_launch(int64_t M, const float* A, const OvhWeight* w, const float* C, int64_t ldc) {
+  if (w->f32 || w->silu_pair || !C || ldc < w->w.N) return false;
+  const int64_t min_rows = ovh::f16_min_rows();
+  if (min_rows > 0 && M >= min_rows) return false;
+  return ovh::linear_small_applies(M, A, w->w, C, ldc);
+}
 }  // namespace
 
 extern "C" {
@@ -794,6 +804,10 @@ int ovh_linear(int64_t M, const float* A, const OvhWeight* w, float* C, int64_t 
   if (M <= 0) return OV_OK;
   if (!w || !A) return fail(OV_ERR_INVALID_ARG, "null argument");
   const hipStream_t st = as_stream(stream);
+  if (linear_one_launch(M, A, w, C, ldc)) {
+    OVH_HIP(ovh::launch_linear_small(M, A, w->w, C, ldc, accumulate != 0, st), "linear launch");
+    return OV_OK;
+  }
   // K a multiple of 128: the codes tile-major (the layout the 16x16 GEMM reads
   // as contiguous 1 KiB tiles), else row-major; the scales [M][Kb] follow at
   // the next 256-byte boundary
