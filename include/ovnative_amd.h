@@ -318,8 +318,8 @@ int ovh_attention(const OvhAttnSegment* segs, int n_segs, int n_heads, int n_kv_
                   int head_dim, const float* q, int64_t q_stride, const float* k, const float* v,
                   int64_t kv_stride, float scale, float* out, int64_t out_stride, void* stream);
 /* The same attention with the products split into f16 hi/lo parts on the f16
- * matrix core (hi*hi + hi*lo + lo*hi, ~2^-22 relative; 5x less matrix-core
- * time than the fp32 form).  No reference counterpart beyond ovh_attention's.
+ * matrix core (hi*hi + hi*lo + lo*hi, ~2^-22 relative; half the matrix-core
+ * time of the fp32 form).  No reference counterpart beyond ovh_attention's.
  * |k| and |v| must stay below 65504 (OV_ERR_INVALID_ARG otherwise); strides a
  * multiple of 8, kv_off a whole number of rows, at most 32 segments.  Allocates
  * its split workspace stream-ordered and synchronises the stream. */

@@ -154,17 +154,19 @@ hipError_t launch_qk_norm_rope(float* q, float* k, const float* qw, const float*
 //
 // Work split: one workgroup per (segment, head, 32 query rows); its 4
 // wavefronts take every 4th block of 32 keys and keep a flash-style running
-// max / sum / output, merged through LDS at the end.  Products run on the fp32
-// matrix core (V_MFMA_F32_32X32X2_F32):
+// max / sum / output, merged through LDS at the end.
 //   * scores are computed transposed, S^T = K · Q^T, so each lane ends up with
 //     16 keys of ONE query (lane % 32); the softmax row statistics are then a
 //     per-lane reduction plus one exchange with lane ^ 32;
 //   * those 16 probabilities are exactly the A operand that P · V needs from
 //     this lane (query = lane % 32, key = the same 16 keys), so P never leaves
 //     registers;
-//   * the head dimension is split so that each lane loads float4s: for scores
-//     lane (r, h) holds d = 8c + 4h + e (c < 16, e < 4) of its key/query row;
-//     for P · V output column j of block c' is d = 4j + c'.
+//   * for P · V output column j of block c' is d = 4j + c', so a lane loads V as
+//     float4s.
+// attention_f32_body below has its products on the fp32 matrix core
+// (V_MFMA_F32_32X32X2_F32; lane (r, h) holds d = 8c + 4h + e (c < 16, e < 4) of
+// its key/query row); attention_kernel has them on the bf16 matrix core and
+// leaves only what that cannot represent to the former.
 // Loads of K, V, Q rows past the segment end are clamped to its last row (and
 // masked out of the softmax / not stored), so every access stays in bounds.
 constexpr int kAttnD = 128;
@@ -172,20 +174,25 @@ constexpr int kAttnQ = 32;   // query rows per workgroup
 constexpr int kAttnK = 32;   // keys per block
 constexpr int kAttnWaves = 4;
 
+constexpr int kQPad = kAttnD + 8;  // LDS row of a Q plane, in halves
+constexpr int kPartRow = kAttnD + 4;  // LDS row of a merge partial, in floats
+// The split forms' lazy softmax reference: a row's exponents are taken
+// against a value at most this far (base 2) below its largest score so far.
+constexpr float kLazyLog2 = 8.0f;
+constexpr float kLog2e = 1.44269504088896340736f;
+constexpr float kMaskedLog2 = -1e29f * kLog2e;
+
 __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
-__global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args) {
-  __shared__ float part[kAttnWaves][kAttnQ][kAttnD];  // per-wave unnormalised outputs
-  __shared__ float mstat[kAttnWaves][kAttnQ], lstat[kAttnWaves][kAttnQ];
-  __shared__ float alpha_s[kAttnWaves][kAttnQ];
-
-  const AttnSeg seg = args.segs[blockIdx.z];
+// (part, mstat, lstat, alpha_s: LDS; part holds per-wave unnormalised outputs)
+__device__ __forceinline__ void attention_f32_body(const AttnArgs& args, const AttnSeg& seg, int h,
+                                                   int q0, float (*part)[kAttnQ][kPartRow],
+                                                   float (*mstat)[kAttnQ], float (*lstat)[kAttnQ],
+                                                   float (*alpha_s)[kAttnQ]) {
   const int S = seg.rows;
-  const int q0 = blockIdx.x * kAttnQ;
-  if (q0 >= S) return;  // uniform for the workgroup
-  const int h = blockIdx.y, kvh = h / args.group;
+  const int kvh = h / args.group;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int r32 = lane & 31, hf = lane >> 5;
 
@@ -326,24 +333,306 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args) {
   }
 }
 
-hipError_t launch_attention(const AttnArgs& args, int max_rows, hipStream_t st) {
-  if (args.n_segs <= 0 || max_rows <= 0) return hipSuccess;
-  const dim3 grid((unsigned)((max_rows + kAttnQ - 1) / kAttnQ), (unsigned)args.n_heads,
-                  (unsigned)args.n_segs);
-  hipLaunchKernelGGL(attention_kernel, grid, dim3(256), 0, st, args);
-  return hipGetLastError();
+// ---------------------------------------------------------------------------
+// The fp32 form on the bf16 matrix core.  x = hi + mid + lo with hi the upper 16
+// bits of x, mid those of x - hi and lo = x - hi - mid: each part is a bf16 and
+// their sum is x exactly (3 x 8 bits), over fp32's whole range.  Six products
+// (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi; the dropped ones are below
+// 2^-24) on V_MFMA_F32_32X32X16_BF16 replace eight V_MFMA_F32_32X32X2_F32: 192
+// against 512 matrix clocks per 32x32x16 product, and fewer roundings (16 k a
+// rounding instead of 2).  The splitting, 5.5 VALU instructions a value, is then
+// what the matrix core overlaps with; K and V are split by the wavefront that
+// uses them, straight from the fp32 rows (no workspace, as before).  Softmax
+// with the lazy reference of the split-f16 form below, but log2(e) multiplied in
+// after the reference is taken away: biases of some hundreds in base 2 doubled
+// the error.
+// What does not split goes to the fp32 products: an infinity or a NaN (inf - inf;
+// it leaves a NaN in the tile's sums) and parts below bf16's range.  Parts lose
+// at most 2^-126: nothing for a score when every q of the tile is 0 or 2^-100 to
+// 2^100 in magnitude, nothing for an output of 2^-100 or more; a workgroup with
+// another q or output, or with a sum that is not finite, works its tile out again.
+// K's next block is fetched in halves: all of it beside all of V spilled 164 B.
+// 16 heads, fp32 products -> these: the call with segments of 700 and 620 rows
+// 110 -> 66 us, 16 x 600 masked rows 603 -> 471, 33 rows 15 (either); error
+// against 64 bits 4.6e-7 -> 4.0e-7 of the result's norm (700 rows), 1.2e-7 ->
+// 1.0e-7 (600 masked).
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ f32x16 mfma_b(b8 a, b8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+struct Parts {
+  b8 hi, mid, lo;
+};
+
+__device__ __forceinline__ Parts split3(const float (&x)[8]) {
+  i32x4 d[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float v0 = x[2 * i], v1 = x[2 * i + 1];
+#pragma unroll
+    for (int part = 0; part < 3; ++part) {
+      const uint32_t u0 = __float_as_uint(v0), u1 = __float_as_uint(v1);
+      d[part][i] = (int)__builtin_amdgcn_perm(u1, u0, 0x07060302u);  // the upper halves
+      if (part < 2) {
+        v0 = __fsub_rn(v0, __uint_as_float(u0 & 0xffff0000u));
+        v1 = __fsub_rn(v1, __uint_as_float(u1 & 0xffff0000u));
+      }
+    }
+  }
+  return Parts{__builtin_bit_cast(b8, d[0]), __builtin_bit_cast(b8, d[1]),
+               __builtin_bit_cast(b8, d[2])};
+}
+
+// c += a b, smallest products first
+__device__ __forceinline__ f32x16 mfma_x6(const Parts& a, const Parts& b, f32x16 c) {
+  c = mfma_b(a.lo, b.hi, c);
+  c = mfma_b(a.hi, b.lo, c);
+  c = mfma_b(a.mid, b.mid, c);
+  c = mfma_b(a.mid, b.hi, c);
+  c = mfma_b(a.hi, b.mid, c);
+  return mfma_b(a.hi, b.hi, c);
+}
+
+__global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qtiles, int per_xcd) {
+  // the Q parts (3 x 32 x kQPad bf16) alias the start of part, as in the split form
+  __shared__ __attribute__((aligned(16))) float part[kAttnWaves][kAttnQ][kPartRow];
+  __shared__ float mstat[kAttnWaves][kAttnQ], lstat[kAttnWaves][kAttnQ];
+  __shared__ float alpha_s[kAttnWaves][kAttnQ];
+  constexpr int kPlane = kAttnQ * kQPad;
+  uint16_t* const qs = reinterpret_cast<uint16_t*>(&part[0][0][0]);
+
+  // XCD-aware task order, as in the split form
+  const int task = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+  if (task >= args.n_segs * args.n_heads * qtiles) return;
+  const int qt = task % qtiles, sh = task / qtiles, sidx = sh / args.n_heads;
+  const int h = sh - sidx * args.n_heads, kvh = h / args.group;
+  const AttnSeg seg = args.segs[sidx];
+  const int S = seg.rows, q0 = qt * kAttnQ;
+  if (q0 >= S) return;  // uniform for the workgroup
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int r32 = lane & 31, hf = lane >> 5;
+  const float* const kb = args.k + seg.kv_off + (int64_t)kvh * kAttnD + 8 * hf;
+  const float* const vb = args.v + seg.kv_off + (int64_t)kvh * kAttnD + 4 * r32;
+
+  // K rows of a block: chunk c = dims 16 c + 8 hf .. +7 of key t0 + r32; V rows:
+  // dims 4 r32 .. +3 of the 16 keys t0 + 8 (i / 4) + 4 hf + i % 4, the keys whose
+  // probabilities this lane holds.  Rows past the segment repeat its last.
+  f32x4 kx[16], vx[16];
+  auto load_k = [&](int t0, int half) __attribute__((always_inline)) {
+    const float* src = kb + (int64_t)min(t0 + r32, S - 1) * args.kv_stride;
+#pragma unroll
+    for (int c = 4 * half; c < 4 * half + 4; ++c) {
+      kx[2 * c] = *reinterpret_cast<const f32x4*>(src + 16 * c);
+      kx[2 * c + 1] = *reinterpret_cast<const f32x4*>(src + 16 * c + 4);
+    }
+  };
+  auto load_v = [&](int t0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int t = min(t0 + 8 * (i >> 2) + 4 * hf + (i & 3), S - 1);
+      vx[i] = *reinterpret_cast<const f32x4*>(vb + (int64_t)t * args.kv_stride);
+    }
+  };
+  const int nblk = (S + kAttnK - 1) / kAttnK;
+  load_k(min(wave, nblk - 1) * kAttnK, 0);
+  load_k(min(wave, nblk - 1) * kAttnK, 1);
+  // ---- Q: 16 values of a row per thread, split into LDS
+  bool odd = false;
+  {
+    const int q_row = threadIdx.x >> 3, q_c0 = (threadIdx.x & 7) * 16;
+    const float* src = args.q + seg.q_off + (int64_t)min(q0 + q_row, S - 1) * args.q_stride +
+                       (int64_t)h * kAttnD + q_c0;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      float x[8];
+      const f32x4 x0 = *reinterpret_cast<const f32x4*>(src + 8 * j);
+      const f32x4 x1 = *reinterpret_cast<const f32x4*>(src + 8 * j + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[e] = x0[e];
+        x[4 + e] = x1[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        odd |= x[e] != 0.f && !(fabsf(x[e]) >= 0x1p-100f && fabsf(x[e]) <= 0x1p100f);
+      const Parts p = split3(x);
+      uint16_t* const dst = qs + q_row * kQPad + q_c0 + 8 * j;
+      *reinterpret_cast<b8*>(dst) = p.hi;
+      *reinterpret_cast<b8*>(dst + kPlane) = p.mid;
+      *reinterpret_cast<b8*>(dst + 2 * kPlane) = p.lo;
+    }
+  }
+  odd = __syncthreads_or(odd);  // uniform
+  const uint16_t* const qr = qs + r32 * kQPad + 8 * hf;
+  const float* const brow = seg.bias ? seg.bias + (int64_t)min(q0 + r32, S - 1) * S : nullptr;
+
+  f32x16 o[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[c][e] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+  for (int blk = odd ? nblk : wave; blk < nblk; blk += kAttnWaves) {
+    const int t0 = blk * kAttnK;
+    // ---- S^T = K Q^T
+    f32x16 st;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) st[e] = 0.f;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      float x[8];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[e] = kx[2 * c][e];
+        x[4 + e] = kx[2 * c + 1][e];
+      }
+      const Parts q{*reinterpret_cast<const b8*>(qr + 16 * c),
+                    *reinterpret_cast<const b8*>(qr + kPlane + 16 * c),
+                    *reinterpret_cast<const b8*>(qr + 2 * kPlane + 16 * c)};
+      st = mfma_x6(split3(x), q, st);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // K's registers are free from here
+    load_v(t0);
+    load_k(min(blk + kAttnWaves, nblk - 1) * kAttnK, 0);
+    // ---- softmax; key of element e is t0 + 8 (e / 4) + 4 hf + e % 4
+    float p[16], bmax = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int t = t0 + 8 * (e >> 2) + 4 * hf + (e & 3);
+      p[e] = __fmul_rn(st[e], args.scale);
+      if (brow) p[e] = __fadd_rn(p[e], brow[min(t, S - 1)]);
+      if (t >= S) p[e] = -INFINITY;
+      bmax = fmaxf(bmax, p[e]);
+    }
+    bmax = fmaxf(bmax, __shfl_xor(bmax, 32));
+    const bool up = bmax > m_run + kLazyLog2 / kLog2e;
+    const float m_new = up ? bmax : m_run;
+    const float m_ref = m_new == -INFINITY ? 0.f : m_new;  // all keys so far at -inf
+    float psum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      p[e] = __builtin_amdgcn_exp2f(__fmul_rn(p[e] - m_ref, kLog2e));
+      psum = __fadd_rn(psum, p[e]);
+    }
+    psum = __fadd_rn(psum, __shfl_xor(psum, 32));
+    const float alpha = __builtin_amdgcn_exp2f(__fmul_rn(m_run - m_ref, kLog2e));
+    l_run = fmaf(l_run, alpha, psum);
+    if (__any(up)) {  // uniform
+      if (hf == 0) alpha_s[wave][r32] = alpha;
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 a4 = *reinterpret_cast<const f32x4*>(&alpha_s[wave][8 * g + 4 * hf]);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[c][4 * g + e] = __fmul_rn(o[c][4 * g + e], a4[e]);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    m_run = m_new;
+    // ---- O += P V: 16-key chunk c takes this lane's p[8 c .. 8 c + 7]
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      float x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = p[8 * c + j];
+      const Parts pp = split3(x);
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = vx[8 * c + j][db];
+        o[db] = mfma_x6(pp, split3(x), o[db]);
+      }
+      if (c == 0) {  // V's first half is used up: room for the rest of K
+        __builtin_amdgcn_sched_barrier(0);
+        load_k(min(blk + kAttnWaves, nblk - 1) * kAttnK, 1);
+      }
+    }
+  }
+
+  __syncthreads();  // every wavefront is done with the Q parts
+  // ---- merge the 4 key splits, as in the split form
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    f32x4 w4;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) w4[c] = o[c][e];
+    *reinterpret_cast<f32x4*>(&part[wave][8 * (e >> 2) + 4 * hf + (e & 3)][4 * r32]) = w4;
+  }
+  if (hf == 0) {
+    mstat[wave][r32] = m_run;
+    lstat[wave][r32] = l_run;
+  }
+  __syncthreads();
+  const int qi = lane & 31, d0 = 32 * wave + 16 * hf;
+  float M = -INFINITY, nan = 0.f;
+#pragma unroll
+  for (int w = 0; w < kAttnWaves; ++w) {
+    M = fmaxf(M, mstat[w][qi]);
+    nan = fmaf(lstat[w][qi], 0.f, nan);
+  }
+  float ov[16];
+  float f[kAttnWaves], L = 0.f;
+#pragma unroll
+  for (int w = 0; w < kAttnWaves; ++w) {
+    f[w] = mstat[w][qi] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(__fmul_rn(mstat[w][qi] - M, kLog2e));
+    L = fmaf(lstat[w][qi], f[w], L);
+  }
+  const float inv = __fdiv_rn(1.f, L);
+#pragma unroll
+  for (int j = 0; j < 16; j += 4) {
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kAttnWaves; ++w) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(&part[w][qi][d0 + j]);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        acc[c] = fmaf(x[c], f[w], acc[c]);
+        nan = fmaf(x[c], 0.f, nan);  // an infinity counts as well
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      ov[j + c] = M < -1e29f ? 0.f : __fmul_rn(acc[c], inv);
+      odd |= ov[j + c] != 0.f && fabsf(ov[j + c]) < 0x1p-100f;
+    }
+  }
+  if (__syncthreads_or(odd || !(nan == 0.f))) {
+    attention_f32_body(args, seg, h, q0, part, mstat, lstat, alpha_s);
+    return;
+  }
+  if (q0 + qi >= S) return;
+  float* const dst =
+      args.out + seg.q_off + (int64_t)(q0 + qi) * args.out_stride + (int64_t)h * kAttnD + d0;
+#pragma unroll
+  for (int j = 0; j < 16; j += 4)
+    *reinterpret_cast<f32x4*>(dst + j) = f32x4{ov[j], ov[j + 1], ov[j + 2], ov[j + 3]};
+}
+
+hipError_t launch_attention(const AttnArgs& args, int max_rows, hipStream_t st) {
+  if (args.n_segs <= 0 || max_rows <= 0) return hipSuccess;
+  const int qtiles = (max_rows + kAttnQ - 1) / kAttnQ;
+  const int64_t per_xcd = ((int64_t)args.n_segs * args.n_heads * qtiles + 7) / 8;
+  if (8 * per_xcd > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(attention_kernel, dim3((unsigned)(8 * per_xcd)), dim3(256), 0, st, args, qtiles,
+                     (int)per_xcd);
+  return hipGetLastError();
+}
 
 // ---------------------------------------------------------------------------
 // Split-f16 attention.  fp32 x = hi + lo with hi = f16(x) and lo = f16(x - hi):
 // hi*hi + hi*lo + lo*hi carries the product to ~2^-22 relative (lo*lo is
 // dropped), and each term is exact in the fp32 accumulator, so three
 // V_MFMA_F32_32X32X16_F16 replace eight V_MFMA_F32_32X32X2_F32 per 32x32x16
-// product: 5.3x less matrix-core time than the fp32 kernel above, same
-// structure otherwise.  Values beyond the f16 range would become inf: the split
-// pass reports them through `overflow` (the reference's own GPU path runs its
-// activations in fp16 too, cuda_lm.cu:1086-1160).
+// product: 5.3x less matrix-core time than fp32 products and half of the
+// kernel's above, same structure otherwise.  Values beyond the f16 range would
+// become inf: the split pass reports them through `overflow` (the reference's
+// own GPU path runs its activations in fp16 too, cuda_lm.cu:1086-1160).
 
 __device__ __forceinline__ f32x16 mfma_h(h8 a, h8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
@@ -569,14 +858,6 @@ __global__ __launch_bounds__(256) void qk_norm_rope_split_kernel(
 // merged through LDS); the Q planes of the workgroup sit in LDS, the softmax
 // runs in base 2 (scores scaled by log2(e), V_EXP_F32), and each wavefront loads
 // the K and V fragments of its next block while it computes the current one.
-constexpr int kQPad = kAttnD + 8;  // LDS row of a Q plane, in halves
-constexpr int kPartRow = kAttnD + 4;  // LDS row of a merge partial, in floats
-// The split forms' lazy softmax reference: a row's exponents are taken
-// against a value at most this far (base 2) below its largest score so far.
-constexpr float kLazyLog2 = 8.0f;
-constexpr float kLog2e = 1.44269504088896340736f;
-constexpr float kMaskedLog2 = -1e29f * kLog2e;
-
 // The mask word of a segment without a mask: every key visible.
 __device__ const uint32_t kAllVisible[1] = {0xffffffffu};
 
