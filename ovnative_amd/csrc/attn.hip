@@ -1245,8 +1245,8 @@ __device__ __forceinline__ bool bias_values(const AttnSplit& sp, int s) {
 
 // The operator's form: a bias that is a mask (every value 0 or -1e30, as the
 // reference builds them) is attended through its bit words, 1/32 of the bytes
-// and with the K/V prefetch the float form has no registers for (2 x 300: 21.4
-// -> 15.2 us); any other through its values.  The same bits either way.
+// and with the K/V prefetch the float form has no registers for (2 x 300: 20.6
+// -> 16.2 us); any other through its values.  The same bits either way.
 __global__ __launch_bounds__(256, 2) void attention_split_auto_kernel(AttnArgs args, AttnSplit sp,
                                                                       int qtiles, int per_xcd) {
   __shared__ __attribute__((aligned(16))) SplitLds lds;
@@ -1566,8 +1566,8 @@ __global__ __launch_bounds__(256, 2) void attention_split_lds_kernel(AttnArgs ar
   attention_split_lds_body<kBits>(args, sp, qtiles, per_xcd, kv0, kv1, xs, ms);
 }
 
-// The operator's form, as attention_split_auto_kernel (16 x 1024, 8 masked: 531
-// -> 420 us; the float form reads each bias row once per head).
+// The operator's form, as attention_split_auto_kernel (16 x 1024, 8 masked: 530
+// -> 441 us; the float form reads each bias row once per head).
 __global__ __launch_bounds__(256, 2) void attention_split_lds_auto_kernel(AttnArgs args,
                                                                           AttnSplit sp, int qtiles,
                                                                           int per_xcd) {

@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256) void f32_split_rows_kernel(int64_t M, int64_t 
 // the row in registers (one pass over it), four rows per workgroup, and the
 // planes go through LDS so that the four rows' 16-byte slots leave as 64
 // contiguous bytes (a row's own stores are 16 bytes in every 512).  M = 600,
-// K = 1024: 7.8 -> 3.6 us.  Rows past M are left alone (see above).
+// K = 1024: 7.9 -> 5.1 us.  Rows past M are left alone (see above).
 template <int P>
 __global__ __launch_bounds__(256) void f32_split_rows_p_kernel(int64_t M,
                                                                const float* __restrict__ A,
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(64) void rmsnorm_split_rows_kernel(const float* __r
 // its 2.5 PFLOP/s).  So stage s + 1's fragments are read into a second register
 // set between the products of stage s, one read after each product; stage s's
 // slot is then free at the barrier that publishes stage s + 1.  M = 600,
-// N = 8200, K = 1024: 47.2 -> 38.3 us (630 -> 787 TFLOP/s of f16 products).
+// N = 8200, K = 1024: 47.2 -> 40.9 us (640 -> 739 TFLOP/s of f16 products).
 __device__ __forceinline__ f32x16 mfma_h(h8 a, h8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }

@@ -1,5 +1,5 @@
 // Skinny-M grouped int8 GEMM (M <= 128): the projections of a layer at short
-// sequence lengths (BASELINE config 2) as one launch that streams each weight
+// sequence lengths as one launch that streams each weight
 // from HBM once, with as many weight bytes in flight as the device holds.
 //
 // Arithmetic: the reference's per-output block epilogue
