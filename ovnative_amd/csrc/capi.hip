@@ -310,6 +310,14 @@ int linear_q_sliced(int64_t M, const int8_t* aq, const float* asc, const OvhWeig
 namespace {
 constexpr int kMaxDevices = 64;
 
+// Set-up calls made once per process: another thread's graph capture in the
+// global mode neither refuses them nor is broken by them.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // A call's workspace, stream-ordered (hipFreeAsync after the last launch): from
 // a pool of the library's own per device, which keeps up to kPoolKeep bytes
 // between calls and gives the rest back at the next synchronisation.  The
@@ -327,6 +335,7 @@ hipMemPool_t call_pool(int dev) {
   std::lock_guard<std::mutex> lock(g_pool_mu);
   if (!g_pool_tried[dev]) {
     g_pool_tried[dev] = true;
+    const RelaxedCapture relaxed;
     hipMemPoolProps props{};
     props.allocType = hipMemAllocationTypePinned;
     props.handleTypes = hipMemHandleTypeNone;
@@ -384,6 +393,7 @@ struct AttnSlot {
     if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
     std::unique_lock<std::mutex> lock(g_attn.mu);
     if (!g_attn.overflow) {
+      const RelaxedCapture relaxed;
       void* p = nullptr;
       e = hipHostMalloc(&p, 64 * kAttnSlots, hipHostMallocPortable);
       if (e != hipSuccess) return e;
