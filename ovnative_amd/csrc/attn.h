@@ -67,16 +67,18 @@ struct AttnSplit {
   int64_t vt_cols;
   int64_t vt_off[kAttnMaxSegs];
   int32_t n_kv_heads;
-  // set non-zero when a |k| or |v| is beyond the f16 range (device memory, or, for
-  // launch_attention_split, pinned host memory)
+  // set non-zero when a |k| or |v| is beyond the f16 range (device memory)
   uint32_t* overflow;
   // launch_attention_split: the distinct biases of the segments, each turned into
   // mask words (AttnSeg::bits points at them) as long as every value is 0 or
-  // -1e30; not_mask[m] = ticket (device memory, never `ticket` before the call)
+  // -1e30; found[m] = ticket (device memory, never `ticket` before the call)
   // where one is not, and the segments of that bias are attended with its values.
-  // mask_of[s]: the bias of segment s, -1 without one.
+  // mask_of[s]: the bias of segment s, -1 without one.  found[kAttnMaxSegs] =
+  // ticket where `overflow` would be set; the attention then sets *report (pinned
+  // host memory, or null).
   uint64_t ticket;
-  uint64_t* not_mask;
+  uint64_t* found;
+  uint32_t* report;
   int32_t n_masks;
   struct {
     const float* bias;

@@ -631,7 +631,7 @@ hipError_t launch_attention(const AttnArgs& args, int max_rows, hipStream_t st) 
 // V_MFMA_F32_32X32X16_F16 replace eight V_MFMA_F32_32X32X2_F32 per 32x32x16
 // product: 5.3x less matrix-core time than fp32 products and half of the
 // kernel's above, same structure otherwise.  Values beyond the f16 range would
-// become inf: the split pass reports them through `overflow` (the reference's
+// become inf: the split pass reports them (the reference's
 // own GPU path runs its activations in fp16 too, cuda_lm.cu:1086-1160).
 
 __device__ __forceinline__ f32x16 mfma_h(h8 a, h8 b, f32x16 c) {
@@ -754,18 +754,20 @@ __device__ __forceinline__ bool mask_row(const float* __restrict__ bias, int row
 // Standalone split of K and V for one attention call: first the masks' bit
 // words, one row per wavefront (a row is a chain of loads, so these start with
 // the launch), then one workgroup per (segment, key tile, KV head, dim quarter).
-// Every row of a bias that is no mask reports it, all with one value to one word
-// and read by the next launch only: a plain store, which the XCD's L2 merges.
-// Stores at agent scope each went through to memory, one after the other (16
-// biases of 600 rows of values: 31 us without the masks' pass, 258 with them,
-// 34 with plain ones).
+// What it finds (a bias that is no mask, a value beyond f16) every row or tile
+// reports with the call's one ticket in one word, read by the next launch only:
+// plain stores, which the XCD's L2 merges.  Stores at agent or system scope each
+// went through to memory or the host, one after the other (16 biases of 600 rows
+// of values: 31 us without the masks' pass, 258 with them, 34 with plain ones;
+// 16 x 600 rows beyond f16: the refused call 3550 -> 240 us).
 __global__ __launch_bounds__(256) void split_kv_kernel(AttnArgs a, AttnSplit sp, int ktiles,
                                                        int64_t mask_jobs) {
   __shared__ float tile[32][33];
   int64_t j = blockIdx.x;
   if (j >= mask_jobs) {
     if (split_v_job(a, sp, j - mask_jobs, ktiles, tile, true))
-      __hip_atomic_store(sp.overflow, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(sp.found + kAttnMaxSegs, sp.ticket, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_WORKGROUP);
     return;
   }
   int m = 0;
@@ -774,7 +776,7 @@ __global__ __launch_bounds__(256) void split_kv_kernel(AttnArgs a, AttnSplit sp,
   if (row >= sp.masks[m].rows) return;
   if (mask_row(sp.masks[m].bias, sp.masks[m].rows, row, sp.masks[m].bits, threadIdx.x & 63) &&
       (threadIdx.x & 63) == 0)
-    __hip_atomic_store(sp.not_mask + m, sp.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_store(sp.found + m, sp.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // The runner's form of qk-norm + RoPE + plane split, in one launch.  The first
@@ -1246,7 +1248,13 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(AttnArgs args, 
 // pass of this call found to be no mask (uniform).
 __device__ __forceinline__ bool bias_values(const AttnSplit& sp, int s) {
   const int m = sp.mask_of[s];
-  return m >= 0 && __builtin_amdgcn_readfirstlane((int)(sp.not_mask[m] == sp.ticket));
+  return m >= 0 && __builtin_amdgcn_readfirstlane((int)(sp.found[m] == sp.ticket));
+}
+
+// A value beyond f16 told to the host, by one thread of the launch.
+__device__ __forceinline__ void report_overflow(const AttnSplit& sp) {
+  if (blockIdx.x == 0 && threadIdx.x == 0 && sp.report && sp.found[kAttnMaxSegs] == sp.ticket)
+    __hip_atomic_store(sp.report, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The operator's form: a bias that is a mask (every value 0 or -1e30, as the
@@ -1262,6 +1270,7 @@ __global__ __launch_bounds__(256, 2) void attention_split_auto_kernel(AttnArgs a
     attention_split_body<false>(args, sp, qtiles, per_xcd, lds);
   else
     attention_split_body<true>(args, sp, qtiles, per_xcd, lds);
+  report_overflow(sp);
 }
 
 // ---------------------------------------------------------------------------
@@ -1585,6 +1594,7 @@ __global__ __launch_bounds__(256, 2) void attention_split_lds_auto_kernel(AttnAr
     attention_split_lds_body<false>(args, sp, qtiles, per_xcd, kv0, kv1, xs, ms);
   else
     attention_split_lds_body<true>(args, sp, qtiles, per_xcd, kv0, kv1, xs, ms);
+  report_overflow(sp);
 }
 #undef OVH_ATTN_LONG_LDS
 

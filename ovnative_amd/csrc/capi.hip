@@ -7,7 +7,6 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
-#include <condition_variable>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -366,59 +365,60 @@ hipError_t call_malloc(void** ptr, size_t bytes, hipStream_t st) {
 }
 
 // What a split-attention call reports while it runs: a pinned host word (|k| or
-// |v| beyond f16) and device words for its biases, one slot per call in flight.
-// The device words compare with the call's ticket, so nothing is cleared between
-// calls (a launch of its own); tickets never repeat.
+// |v| beyond f16) and device words (what it found, AttnSplit::found), one slot per
+// call in flight.  The device words compare with the call's ticket, so nothing is
+// cleared between calls (a launch of its own); tickets never repeat.  A call that
+// finds every slot in use waits for none of them: it has its words in its
+// workspace, cleared, and copies the one it needs.
 constexpr int kAttnSlots = 32;
-__device__ uint64_t attn_not_mask[kAttnSlots][ovh::kAttnMaxSegs];
+constexpr int kAttnFound = ovh::kAttnMaxSegs + 1;
+__device__ uint64_t attn_found[kAttnSlots][kAttnFound];
 struct AttnSlots {
   std::mutex mu;
-  std::condition_variable freed;
   uint32_t busy = 0;               // bit per slot
-  uint32_t* overflow = nullptr;    // pinned, [kAttnSlots], one word per 64 bytes
-  uint64_t* not_mask[kMaxDevices] = {};
+  uint32_t* report = nullptr;      // pinned, [kAttnSlots], one word per 64 bytes
+  uint64_t* found[kMaxDevices] = {};
   uint64_t ticket = 0;
 };
 AttnSlots g_attn;
 
 struct AttnSlot {
-  int i = -1;
-  volatile uint32_t* overflow = nullptr;
-  uint64_t* not_mask = nullptr;
+  int i = -1;  // -1 after take(): none was free
+  volatile uint32_t* report = nullptr;
+  uint64_t* found = nullptr;
   uint64_t ticket = 0;
   hipError_t take() {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
-    std::unique_lock<std::mutex> lock(g_attn.mu);
-    if (!g_attn.overflow) {
+    std::lock_guard<std::mutex> lock(g_attn.mu);
+    ticket = ++g_attn.ticket;
+    if (g_attn.busy == ~0u) return hipSuccess;
+    if (!g_attn.report) {
       const RelaxedCapture relaxed;
       void* p = nullptr;
       e = hipHostMalloc(&p, 64 * kAttnSlots, hipHostMallocPortable);
       if (e != hipSuccess) return e;
-      g_attn.overflow = static_cast<uint32_t*>(p);
+      g_attn.report = static_cast<uint32_t*>(p);
     }
-    if (!g_attn.not_mask[dev]) {
+    if (!g_attn.found[dev]) {
       void* p = nullptr;
-      e = hipGetSymbolAddress(&p, HIP_SYMBOL(attn_not_mask));
+      e = hipGetSymbolAddress(&p, HIP_SYMBOL(attn_found));
       if (e != hipSuccess) return e;
-      g_attn.not_mask[dev] = static_cast<uint64_t*>(p);
+      g_attn.found[dev] = static_cast<uint64_t*>(p);
     }
-    g_attn.freed.wait(lock, [] { return g_attn.busy != ~0u; });
     i = __builtin_ctz(~g_attn.busy);
     g_attn.busy |= 1u << i;
-    overflow = g_attn.overflow + 16 * i;
-    *overflow = 0;
-    not_mask = g_attn.not_mask[dev] + i * ovh::kAttnMaxSegs;
-    ticket = ++g_attn.ticket;
+    report = g_attn.report + 16 * i;
+    *report = 0;
+    found = g_attn.found[dev] + i * kAttnFound;
     return hipSuccess;
   }
   ~AttnSlot() {
     if (i < 0) return;
     std::lock_guard<std::mutex> lock(g_attn.mu);
     g_attn.busy &= ~(1u << i);
-    g_attn.freed.notify_one();
   }
 };
 }  // namespace
@@ -1130,27 +1130,33 @@ int ovh_attention_split(const OvhAttnSegment* segs, int n_segs, int n_heads, int
   const size_t vbytes = sizeof(_Float16) * (size_t)((int64_t)n_kv_heads * head_dim * sp.vt_cols);
   const size_t kbytes = vbytes;  // K and V planes are both tile-major over the padded keys
   char* ws = nullptr;
-  const size_t total = 2 * kbytes + 2 * vbytes + sizeof(uint32_t) * mask_words + 256;
   AttnSlot slot;
   OVH_HIP(slot.take(), "attention_split report slot");
+  const size_t found_bytes = slot.i < 0 ? sizeof(uint64_t) * kAttnFound : 0;
+  const size_t planes = 2 * kbytes + 2 * vbytes;  // a multiple of 256
+  const size_t total = planes + found_bytes + sizeof(uint32_t) * mask_words + 256;
   OVH_HIP(call_malloc(reinterpret_cast<void**>(&ws), total, st), "workspace of attention_split");
   sp.kh = reinterpret_cast<_Float16*>(ws);
   sp.kl = reinterpret_cast<_Float16*>(ws + kbytes);
   sp.vh = reinterpret_cast<_Float16*>(ws + 2 * kbytes);
   sp.vl = reinterpret_cast<_Float16*>(ws + 2 * kbytes + vbytes);
-  uint32_t* const words = reinterpret_cast<uint32_t*>(ws + 2 * kbytes + 2 * vbytes);
+  uint32_t* const words = reinterpret_cast<uint32_t*>(ws + planes + found_bytes);
   for (int m = 0; m < sp.n_masks; ++m) sp.masks[m].bits = words + mask_at[m];
   for (int s = 0; s < n_segs; ++s)
     if (sp.mask_of[s] >= 0) a.segs[s].bits = sp.masks[sp.mask_of[s]].bits;
-  sp.overflow = const_cast<uint32_t*>(slot.overflow);
+  sp.report = const_cast<uint32_t*>(slot.report);
   sp.ticket = slot.ticket;
-  sp.not_mask = slot.not_mask;
-  hipError_t e = ovh::launch_attention_split(a, sp, max_rows, st);
+  sp.found = slot.i < 0 ? reinterpret_cast<uint64_t*>(ws + planes) : slot.found;
+  hipError_t e = slot.i < 0 ? hipMemsetAsync(sp.found, 0, found_bytes, st) : hipSuccess;
+  if (e == hipSuccess) e = ovh::launch_attention_split(a, sp, max_rows, st);
+  uint64_t over = 0;
+  if (e == hipSuccess && slot.i < 0)
+    e = hipMemcpyAsync(&over, sp.found + ovh::kAttnMaxSegs, sizeof over, hipMemcpyDeviceToHost, st);
   (void)hipFreeAsync(ws, st);
   const hipError_t es = hipStreamSynchronize(st);
   if (e == hipSuccess) e = es;
   if (e != hipSuccess) return hip_fail(e, "attention_split");
-  const uint32_t flag = *slot.overflow;
+  const bool flag = slot.i < 0 ? over == sp.ticket : *slot.report != 0;
   if (flag)
     return fail(OV_ERR_INVALID_ARG, "attention_split: |k| or |v| beyond the f16 range; use "
                                     "ovh_attention");

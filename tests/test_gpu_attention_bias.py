@@ -135,3 +135,65 @@ def test_value_biases_cost():
                 ov.attention(q, k, v, segs, 16, 8, split=True)  # returns when done
             times.setdefault(name, []).append(time.perf_counter() - t)
     assert np.median(times["valued"]) <= 2.0 * np.median(times["plain"]), times
+
+
+def test_refusal_cost():
+    """A call whose every K is beyond f16 is refused in at most three times the time
+    of the accepted call (20 times while every tile told the host), and the calls
+    after it are accepted."""
+    import time
+    import ovnative_amd as ov
+    n, rows = 16, 600
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (torch.randn((n * rows, w * D), generator=g).cuda() for w in (16, 8, 8))
+    far = k * 1e7
+    segs = [(None, rows, i * rows, i * rows) for i in range(n)]
+    want = ov.attention(q, k, v, segs, 16, 8, split=True)
+    times = {"taken": [], "refused": []}
+    for _ in range(12):
+        t = time.perf_counter()
+        got = ov.attention(q, k, v, segs, 16, 8, split=True)
+        times["taken"].append(time.perf_counter() - t)
+        assert torch.equal(got, want)
+        t = time.perf_counter()
+        with pytest.raises(ov.InvalidArgument):
+            ov.attention(q, far, v, segs, 16, 8, split=True)
+        times["refused"].append(time.perf_counter() - t)
+    assert np.median(times["refused"]) <= 3 * np.median(times["taken"]), times
+
+
+def test_more_calls_than_report_slots():
+    """40 threads with a call in flight each (a call finds one of 32 report slots,
+    or reports through its own workspace): masks, values and refusals as alone."""
+    import threading
+    import ovnative_amd as ov
+    g = torch.Generator().manual_seed(4)
+    rows = 300
+    mask, other = _mask(g, rows), torch.randn((rows, rows), generator=g).cuda()
+    q, k, v = (torch.randn((2 * rows, n * D), generator=g).cuda() for n in (NH, NKV, NKV))
+    far = k.clone()
+    far[rows + 7, 9] = 1e6
+    segs = [(mask, rows, 0, 0), (other, rows, rows, rows)]
+    want = ov.attention(q, k, v, segs, NH, NKV, split=True)
+    torch.cuda.synchronize()
+    errors, start = [], threading.Barrier(40)
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                start.wait(60)
+                for _ in range(10):
+                    if i % 5 == 1:
+                        with pytest.raises(ov.InvalidArgument):
+                            ov.attention(q, far, v, segs, NH, NKV, split=True)
+                    else:
+                        assert torch.equal(ov.attention(q, k, v, segs, NH, NKV, split=True), want)
+        except BaseException as e:  # noqa: BLE001 - reported by the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(40)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors[0]
