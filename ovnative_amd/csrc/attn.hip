@@ -334,11 +334,15 @@ __device__ __forceinline__ void attention_f32_body(const AttnArgs& args, const A
 }
 
 // ---------------------------------------------------------------------------
-// The fp32 form on the bf16 matrix core.  x = hi + mid + lo with hi the upper 16
-// bits of x, mid those of x - hi and lo = x - hi - mid: each part is a bf16 and
-// their sum is x exactly (3 x 8 bits), over fp32's whole range.  Six products
-// (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi; the dropped ones are below
-// 2^-24) on V_MFMA_F32_32X32X16_BF16 replace eight V_MFMA_F32_32X32X2_F32: 192
+// The fp32 form on the bf16 matrix core.  x = hi + mid + lo with hi = bf16(x),
+// mid = bf16(x - hi) and lo = x - hi - mid: rounded to nearest, mid is at most
+// 2^-8 of x's power of two and lo 2^-17, both of either sign, and the remainder
+// after mid has 8 bits or fewer, so that the sum of the parts is x exactly, over
+// fp32's whole range.  Six products (hi hi, hi mid, mid hi, mid mid, hi lo, lo
+// hi) carry x y: mid lo + lo mid + lo lo are at most 2^-24 of it, and of no one
+// sign.  (Parts cut off instead of rounded leave up to 2^-21, always towards
+// zero: the results shrank by 8e-8 of their root mean square.)  On
+// V_MFMA_F32_32X32X16_BF16 the six replace eight V_MFMA_F32_32X32X2_F32: 192
 // against 512 matrix clocks per 32x32x16 product, and fewer roundings (16 k a
 // rounding instead of 2).  The splitting, 5.5 VALU instructions a value, is then
 // what the matrix core overlaps with; K and V are split by the wavefront that
@@ -352,10 +356,9 @@ __device__ __forceinline__ void attention_f32_body(const AttnArgs& args, const A
 // 2^100 in magnitude, nothing for an output of 2^-100 or more; a workgroup with
 // another q or output, or with a sum that is not finite, works its tile out again.
 // K's next block is fetched in halves: all of it beside all of V spilled 164 B.
-// 16 heads, fp32 products -> these: the call with segments of 700 and 620 rows
-// 110 -> 66 us, 16 x 600 masked rows 603 -> 471, 33 rows 15 (either); error
-// against 64 bits 4.6e-7 -> 4.0e-7 of the result's norm (700 rows), 1.2e-7 ->
-// 1.0e-7 (600 masked).
+// 16 heads, fp32 products -> these: the call with 2 segments of 700 rows 105 ->
+// 69 us, 16 x 600 rows 523 -> 350, masked 594 -> 436, 33 rows 15 (either); error
+// against 64 bits 5.0e-7 -> 4.1e-7 of the result's norm (700 rows).
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ f32x16 mfma_b(b8 a, b8 b, f32x16 c) {
@@ -367,17 +370,19 @@ struct Parts {
 };
 
 __device__ __forceinline__ Parts split3(const float (&x)[8]) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
   i32x4 d[3];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    float v0 = x[2 * i], v1 = x[2 * i + 1];
+    f32x2 v = {x[2 * i], x[2 * i + 1]};
 #pragma unroll
     for (int part = 0; part < 3; ++part) {
-      const uint32_t u0 = __float_as_uint(v0), u1 = __float_as_uint(v1);
-      d[part][i] = (int)__builtin_amdgcn_perm(u1, u0, 0x07060302u);  // the upper halves
+      const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, b2));
+      d[part][i] = (int)u;
       if (part < 2) {
-        v0 = __fsub_rn(v0, __uint_as_float(u0 & 0xffff0000u));
-        v1 = __fsub_rn(v1, __uint_as_float(u1 & 0xffff0000u));
+        v[0] = __fsub_rn(v[0], __uint_as_float(u << 16));
+        v[1] = __fsub_rn(v[1], __uint_as_float(u & 0xffff0000u));
       }
     }
   }
