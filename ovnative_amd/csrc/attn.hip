@@ -347,18 +347,20 @@ __device__ __forceinline__ void attention_f32_body(const AttnArgs& args, const A
 // rounding instead of 2).  The splitting, 5.5 VALU instructions a value, is then
 // what the matrix core overlaps with; K and V are split by the wavefront that
 // uses them, straight from the fp32 rows (no workspace, as before).  Softmax
-// with the lazy reference of the split-f16 form below, but log2(e) multiplied in
-// after the reference is taken away: biases of some hundreds in base 2 doubled
-// the error.
+// with the lazy reference of the split-f16 form below, in base e (biases of some
+// hundreds in base 2 doubled the error).
 // What does not split goes to the fp32 products: an infinity or a NaN (inf - inf;
 // it leaves a NaN in the tile's sums) and parts below bf16's range.  Parts lose
 // at most 2^-126: nothing for a score when every q of the tile is 0 or 2^-100 to
-// 2^100 in magnitude, nothing for an output of 2^-100 or more; a workgroup with
-// another q or output, or with a sum that is not finite, works its tile out again.
+// 2^100 in magnitude, nothing for an output of 2^-100 or more (the probabilities
+// are held times 2^64); a workgroup with another q or output, or with a sum that
+// is not finite, works its tile out again.
 // K's next block is fetched in halves: all of it beside all of V spilled 164 B.
 // 16 heads, fp32 products -> these: the call with 2 segments of 700 rows 105 ->
-// 69 us, 16 x 600 rows 523 -> 350, masked 594 -> 436, 33 rows 15 (either); error
-// against 64 bits 5.0e-7 -> 4.1e-7 of the result's norm (700 rows).
+// 69 us, 16 x 600 rows 522 -> 352, masked 595 -> 438, 2 x 200 17.4 -> 17.2, 33 rows
+// 15 (either); error against 64 bits 5.0e-7 -> 4.1e-7 of the result's norm (700
+// rows).  Rows are addressed with 32-bit offsets (24-bit products): 64-bit ones
+// per lane took 2 x 700 rows 4 us longer.
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ f32x16 mfma_b(b8 a, b8 b, f32x16 c) {
@@ -400,6 +402,21 @@ __device__ __forceinline__ f32x16 mfma_x6(const Parts& a, const Parts& b, f32x16
   return mfma_b(a.hi, b.hi, c);
 }
 
+// 2^64 e^x for x <= 16 to fp32's precision (exp2f of the rounded x log2(e) has up to
+// 15 units of 2^-24 at x = -16): n = rint(x log2(e)), the rest in two fmas with
+// log2(e)'s two parts and by the hardware's 2^y, and 2^(n + 64) added to the
+// exponent.  2^64: the parts of the smallest probability stay in bf16's range; V
+// beyond 2^50 then overflows the sums, and the tile goes to the fp32 products.  0
+// below e^-131 (fp32's own end is e^-104); a NaN stays one.
+__device__ __forceinline__ float exp_p64(float x) {
+  constexpr float kRound = 12582912.f + 64.f;  // 1.5 2^23 + 64
+  constexpr float kLog2eLow = 0x1.4ae0cp-26f;
+  const float u = fmaf(x, kLog2e, kRound), n = __fsub_rn(u, kRound);
+  const float e = __builtin_amdgcn_exp2f(fmaf(x, kLog2eLow, fmaf(x, kLog2e, -n)));
+  const float p = __uint_as_float(__float_as_uint(e) + (__float_as_uint(u) << 23));
+  return x < -131.f ? 0.f : p;
+}
+
 __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qtiles, int per_xcd) {
   // the Q parts (3 x 32 x kQPad bf16) alias the start of part, as in the split form
   __shared__ __attribute__((aligned(16))) float part[kAttnWaves][kAttnQ][kPartRow];
@@ -418,33 +435,42 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qt
   if (q0 >= S) return;  // uniform for the workgroup
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int r32 = lane & 31, hf = lane >> 5;
-  const float* const kb = args.k + seg.kv_off + (int64_t)kvh * kAttnD + 8 * hf;
-  const float* const vb = args.v + seg.kv_off + (int64_t)kvh * kAttnD + 4 * r32;
+  const char* const kb = reinterpret_cast<const char*>(args.k + seg.kv_off + (int64_t)kvh * kAttnD);
+  const char* const vb = reinterpret_cast<const char*>(args.v + seg.kv_off + (int64_t)kvh * kAttnD);
+  // A row's bytes from the segment's first: 24-bit factors and a 32-bit product, or
+  // the fp32 products below, which count in 64 bits.
+  const uint32_t row_bytes = 4 * (uint32_t)args.kv_stride;
+  const bool small = S < 1 << 24 && args.kv_stride < 1 << 22 &&
+                     4 * args.kv_stride * S < (int64_t)0xffff0000;
+  auto row_at = [&](int t) __attribute__((always_inline)) {
+    return (uint32_t)__umul24((uint32_t)min(t, S - 1), row_bytes);
+  };
 
   // K rows of a block: chunk c = dims 16 c + 8 hf .. +7 of key t0 + r32; V rows:
   // dims 4 r32 .. +3 of the 16 keys t0 + 8 (i / 4) + 4 hf + i % 4, the keys whose
   // probabilities this lane holds.  Rows past the segment repeat its last.
   f32x4 kx[16], vx[16];
   auto load_k = [&](int t0, int half) __attribute__((always_inline)) {
-    const float* src = kb + (int64_t)min(t0 + r32, S - 1) * args.kv_stride;
+    const char* const src = kb + (row_at(t0 + r32) + 32 * hf);
 #pragma unroll
     for (int c = 4 * half; c < 4 * half + 4; ++c) {
-      kx[2 * c] = *reinterpret_cast<const f32x4*>(src + 16 * c);
-      kx[2 * c + 1] = *reinterpret_cast<const f32x4*>(src + 16 * c + 4);
+      kx[2 * c] = *reinterpret_cast<const f32x4*>(src + 64 * c);
+      kx[2 * c + 1] = *reinterpret_cast<const f32x4*>(src + 64 * c + 16);
     }
   };
   auto load_v = [&](int t0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int t = min(t0 + 8 * (i >> 2) + 4 * hf + (i & 3), S - 1);
-      vx[i] = *reinterpret_cast<const f32x4*>(vb + (int64_t)t * args.kv_stride);
-    }
+    for (int i = 0; i < 16; ++i)
+      vx[i] = *reinterpret_cast<const f32x4*>(
+          vb + (row_at(t0 + 8 * (i >> 2) + 4 * hf + (i & 3)) + 16 * r32));
   };
   const int nblk = (S + kAttnK - 1) / kAttnK;
-  load_k(min(wave, nblk - 1) * kAttnK, 0);
-  load_k(min(wave, nblk - 1) * kAttnK, 1);
+  if (small) {
+    load_k(min(wave, nblk - 1) * kAttnK, 0);
+    load_k(min(wave, nblk - 1) * kAttnK, 1);
+  }
   // ---- Q: 16 values of a row per thread, split into LDS
-  bool odd = false;
+  bool odd = !small;
   {
     const int q_row = threadIdx.x >> 3, q_c0 = (threadIdx.x & 7) * 16;
     const float* src = args.q + seg.q_off + (int64_t)min(q0 + q_row, S - 1) * args.q_stride +
@@ -505,12 +531,16 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qt
     float p[16], bmax = -INFINITY;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const int t = t0 + 8 * (e >> 2) + 4 * hf + (e & 3);
       p[e] = __fmul_rn(st[e], args.scale);
-      if (brow) p[e] = __fadd_rn(p[e], brow[min(t, S - 1)]);
-      if (t >= S) p[e] = -INFINITY;
-      bmax = fmaxf(bmax, p[e]);
+      if (brow) p[e] = __fadd_rn(p[e], brow[min(t0 + 8 * (e >> 2) + 4 * hf + (e & 3), S - 1)]);
     }
+    if (t0 + kAttnK > S) {  // uniform: keys past the segment
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (t0 + 8 * (e >> 2) + 4 * hf + (e & 3) >= S) p[e] = -INFINITY;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) bmax = fmaxf(bmax, p[e]);
     bmax = fmaxf(bmax, __shfl_xor(bmax, 32));
     const bool up = bmax > m_run + kLazyLog2 / kLog2e;
     const float m_new = up ? bmax : m_run;
@@ -518,13 +548,13 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qt
     float psum = 0.f;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      p[e] = __builtin_amdgcn_exp2f(__fmul_rn(p[e] - m_ref, kLog2e));
+      p[e] = exp_p64(p[e] - m_ref);
       psum = __fadd_rn(psum, p[e]);
     }
     psum = __fadd_rn(psum, __shfl_xor(psum, 32));
-    const float alpha = __builtin_amdgcn_exp2f(__fmul_rn(m_run - m_ref, kLog2e));
-    l_run = fmaf(l_run, alpha, psum);
-    if (__any(up)) {  // uniform
+    float alpha = 1.f;
+    if (__any(up && m_run > -INFINITY)) {  // uniform; before, sum and output are 0
+      alpha = expf(m_run - m_ref);
       if (hf == 0) alpha_s[wave][r32] = alpha;
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -539,6 +569,7 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qt
       }
       __builtin_amdgcn_wave_barrier();
     }
+    l_run = fmaf(l_run, alpha, psum);
     m_run = m_new;
     // ---- O += P V: 16-key chunk c takes this lane's p[8 c .. 8 c + 7]
 #pragma unroll
@@ -585,7 +616,7 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qt
   float f[kAttnWaves], L = 0.f;
 #pragma unroll
   for (int w = 0; w < kAttnWaves; ++w) {
-    f[w] = mstat[w][qi] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(__fmul_rn(mstat[w][qi] - M, kLog2e));
+    f[w] = mstat[w][qi] == -INFINITY ? 0.f : expf(mstat[w][qi] - M);
     L = fmaf(lstat[w][qi], f[w], L);
   }
   const float inv = __fdiv_rn(1.f, L);
@@ -604,7 +635,7 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qt
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       ov[j + c] = M < -1e29f ? 0.f : __fmul_rn(acc[c], inv);
-      odd |= ov[j + c] != 0.f && fabsf(ov[j + c]) < 0x1p-100f;
+      odd |= ov[j + c] != 0.f && !(fabsf(ov[j + c]) >= 0x1p-100f && fabsf(ov[j + c]) < INFINITY);
     }
   }
   if (__syncthreads_or(odd || !(nan == 0.f))) {

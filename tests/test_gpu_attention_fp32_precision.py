@@ -54,3 +54,67 @@ def test_no_error_of_one_sign(rows):
     got, want = _run(q, k, v.abs())
     bias = ((got - want) * want.sign()).mean() / want.square().mean().sqrt()
     assert abs(float(bias)) <= 2.5e-8
+
+
+def _two_keys(scores, values):
+    """Row i and head h attend to key 0 with score 0 and to key 1 with score
+    scores[i, h], both exact in fp32; `values` are those keys' rows of v."""
+    rows = scores.shape[0]
+    q = torch.zeros((rows, NH, D), device="cuda")
+    q[:, :, 0], q[:, :, 1] = scores, 1.0
+    k, v = torch.zeros((rows, NKV, D), device="cuda"), torch.zeros((rows, NKV, D), device="cuda")
+    k[1, :, 0] = 1.0
+    k[2:, :, 1] = -1000.0  # no weight
+    v[0], v[1] = values
+    return q.view(rows, -1), k.view(rows, -1), v.view(rows, -1)
+
+
+@pytest.mark.parametrize("top", [0.0, -4.0, -10.0, -20.0, -40.0])
+def test_probabilities(top):
+    """e^x, x down to -60, to fp32's precision: the hardware's 2^y is good to one
+    unit (2^-23), the quotient and the products round four times more by 2^-24; the
+    argument's own rounding (up to 2^-24 |x|) must not come on top."""
+    g = torch.Generator().manual_seed(int(-top))
+    scores = (top - 20 * torch.rand((512, NH), generator=g)).cuda()
+    got, want = _run(*_two_keys(scores, (0.0, 1.0)), scale=1.0)
+    assert float(((got - want).abs() / want).max()) <= 3.6e-7
+
+
+@pytest.mark.parametrize("below,e", [(60, 49), (60, 53), (60, 80), (80, 110), (83, 119), (86.5, 124),
+                                     (88, 126)])
+def test_small_probability_of_a_large_value(below, e):
+    """A probability of e^-below beside a value of 2^e: their product counts.  Below
+    2^-126 fp32 itself has only 2^-149 / p of the probability left."""
+    g = torch.Generator().manual_seed(e)
+    small, large = 1 + torch.rand((D,), generator=g), 2.0 ** e * (1 + 0.5 * torch.rand((D,), generator=g))
+    scores = torch.full((64, NH), -float(below), device="cuda")
+    got, want = _run(*_two_keys(scores, (small.cuda(), large.cuda())), scale=1.0)
+    assert float(((got - want).abs() / want).max()) <= 3.6e-7 + 2.0 ** -149 / 2.71828 ** -below
+
+
+@pytest.mark.parametrize("e", [30, 45, 49, 50, 51, 52, 53, 54, 55, 56, 57, 58, 60, 64])
+def test_values_at_the_end_of_the_sums(e):
+    """Values of 2^e on both sides of where the sums overflow (and the tile is worked
+    out with fp32 products)."""
+    q, k, v = _inputs(e, 200)
+    got, want = _run(q, k, v.abs() * 2.0 ** e)
+    assert (got - want).norm() <= 1e-6 * want.norm()
+
+
+@pytest.mark.parametrize("rows,stride", [(3, (1 << 22) - 4), (3, 1 << 22), (1000, 1 << 20),
+                                         (1023, 1 << 20), (1025, 1 << 20)])
+def test_far_rows(rows, stride):
+    """Rows of K and V far apart: both sides of the 24-bit row strides and 32-bit
+    offsets of the tile's loads; the bits of the same rows close together, within
+    one rounding where the fp32 products take over."""
+    import ovnative_amd as ov
+    q, k, v = _inputs(rows, rows)
+    near = ov.attention(q, k, v, [(None, rows, 0, 0)], NH, NKV)
+    far = []
+    for t in (k, v):
+        wide = torch.zeros((rows, stride), device="cuda")
+        wide[:, :NKV * D] = t
+        far.append(wide)
+    got = ov.attention(q, *far, [(None, rows, 0, 0)], NH, NKV)
+    assert (got - near).norm() <= 1e-6 * near.norm()
+    assert bool(torch.isfinite(got).all())
