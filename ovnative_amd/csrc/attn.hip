@@ -350,11 +350,14 @@ __device__ __forceinline__ void attention_f32_body(const AttnArgs& args, const A
 // with the lazy reference of the split-f16 form below, in base e (biases of some
 // hundreds in base 2 doubled the error).
 // What does not split goes to the fp32 products: an infinity or a NaN (inf - inf;
-// it leaves a NaN in the tile's sums) and parts below bf16's range.  Parts lose
-// at most 2^-126: nothing for a score when every q of the tile is 0 or 2^-100 to
-// 2^100 in magnitude, nothing for an output of 2^-100 or more (the probabilities
-// are held times 2^64); a workgroup with another q or output, or with a sum that
-// is not finite, works its tile out again.
+// it leaves a NaN in the tile's sums) and parts below bf16's range.  Parts lose at
+// most 2^-126.  That is nothing for the scores when every q of the tile is 0 or at
+// least 2^-100 in magnitude (q loses nothing) and at most 2^90 / max(1, |scale|) (K
+// moves a score by at most 128 2^-126 2^90 = 2^-29); |scale| from 2^-30 on, so that
+// a product too large for fp32 is one too large for a softmax.  And it is nothing
+// for an output of 2^-100 or more (the probabilities are held times 2^64).  A
+// workgroup with another q, scale or output, or with a sum that is not finite,
+// works its tile out again.
 // K's next block is fetched in halves: all of it beside all of V spilled 164 B.
 // 16 heads, fp32 products -> these: the call with 2 segments of 700 rows 105 ->
 // 69 us, 16 x 600 rows 522 -> 352, masked 595 -> 438, 2 x 200 17.4 -> 17.2, 33 rows
@@ -470,7 +473,8 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qt
     load_k(min(wave, nblk - 1) * kAttnK, 1);
   }
   // ---- Q: 16 values of a row per thread, split into LDS
-  bool odd = !small;
+  const float as = fabsf(args.scale), q_max = 0x1p90f / fmaxf(as, 1.f);
+  bool odd = !small || !(as >= 0x1p-30f && as <= 0x1p60f);
   {
     const int q_row = threadIdx.x >> 3, q_c0 = (threadIdx.x & 7) * 16;
     const float* src = args.q + seg.q_off + (int64_t)min(q0 + q_row, S - 1) * args.q_stride +
@@ -487,7 +491,7 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qt
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e)
-        odd |= x[e] != 0.f && !(fabsf(x[e]) >= 0x1p-100f && fabsf(x[e]) <= 0x1p100f);
+        odd |= x[e] != 0.f && !(fabsf(x[e]) >= 0x1p-100f && fabsf(x[e]) <= q_max);
       const Parts p = split3(x);
       uint16_t* const dst = qs + q_row * kQPad + q_c0 + 8 * j;
       *reinterpret_cast<b8*>(dst) = p.hi;

@@ -101,6 +101,18 @@ def test_values_at_the_end_of_the_sums(e):
     assert (got - want).norm() <= 1e-6 * want.norm()
 
 
+@pytest.mark.parametrize("e", [-120, -80, -31, -29, -20, 20, 60, 61, 80, 100, 120])
+@pytest.mark.parametrize("where", ["q", "k"])
+def test_scales(e, where):
+    """A scale of 2^e with Q or K of 2^-e: the same scores, whichever parts that
+    takes out of bf16's range."""
+    q, k, v = _inputs(abs(e), 200)
+    small = 2.0 ** -e
+    got, want = _run(q * small if where == "q" else q, k * small if where == "k" else k, v,
+                     scale=D ** -0.5 * 2.0 ** e)
+    assert (got - want).norm() <= 1e-6 * want.norm()
+
+
 @pytest.mark.parametrize("rows,stride", [(3, (1 << 22) - 4), (3, 1 << 22), (1000, 1 << 20),
                                          (1023, 1 << 20), (1025, 1 << 20)])
 def test_far_rows(rows, stride):
