@@ -355,9 +355,12 @@ __device__ __forceinline__ void attention_f32_body(const AttnArgs& args, const A
 // least 2^-100 in magnitude (q loses nothing) and at most 2^90 / max(1, |scale|) (K
 // moves a score by at most 128 2^-126 2^90 = 2^-29); |scale| from 2^-30 on, so that
 // a product too large for fp32 is one too large for a softmax.  And it is nothing
-// for an output of 2^-100 or more (the probabilities are held times 2^64).  A
-// workgroup with another q, scale or output, or with a sum that is not finite,
-// works its tile out again.
+// for an output of 2^-100 or more (the probabilities are held times 2^64), nor for
+// a zero over V without subnormals.  A workgroup with another q, scale or output,
+// or with a sum that is not finite, works its tile out again: with a NaN in K or V,
+// say, every tile of that KV head, 1.5 to 1.6 times the fp32 products' time; the
+// look for subnormals where a column of V is all zeros makes the call 2 x 700 98 us
+// instead of 70.
 // K's next block is fetched in halves: all of it beside all of V spilled 164 B.
 // 16 heads, fp32 products -> these: the call with 2 segments of 700 rows 105 ->
 // 69 us, 16 x 600 rows 522 -> 352, masked 595 -> 438, 2 x 200 17.4 -> 17.2, 33 rows
@@ -610,6 +613,7 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qt
   }
   __syncthreads();
   const int qi = lane & 31, d0 = 32 * wave + 16 * hf;
+  bool zero = false;
   float M = -INFINITY, nan = 0.f;
 #pragma unroll
   for (int w = 0; w < kAttnWaves; ++w) {
@@ -640,9 +644,22 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qt
     for (int c = 0; c < 4; ++c) {
       ov[j + c] = M < -1e29f ? 0.f : __fmul_rn(acc[c], inv);
       odd |= ov[j + c] != 0.f && !(fabsf(ov[j + c]) >= 0x1p-100f && fabsf(ov[j + c]) < INFINITY);
+      zero |= ov[j + c] == 0.f && M >= -1e29f;
     }
   }
-  if (__syncthreads_or(odd || !(nan == 0.f))) {
+  odd = __syncthreads_or(odd || !(nan == 0.f));
+  // A zero: there is nothing in the column, or only values below 2^-126, which the
+  // matrix core takes for zeros.  The segment's V tells.
+  if (!odd && __syncthreads_or(zero)) {
+    bool tiny = false;
+    for (int t = threadIdx.x >> 5; t < S; t += 8) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(vb + (row_at(t) + 16 * (threadIdx.x & 31)));
+#pragma unroll
+      for (int c = 0; c < 4; ++c) tiny |= x[c] != 0.f && fabsf(x[c]) < 0x1p-126f;
+    }
+    odd = __syncthreads_or(tiny);
+  }
+  if (odd) {
     attention_f32_body(args, seg, h, q0, part, mstat, lstat, alpha_s);
     return;
   }

@@ -113,6 +113,27 @@ def test_scales(e, where):
     assert (got - want).norm() <= 1e-6 * want.norm()
 
 
+@pytest.mark.parametrize("e", [-127, -130, -135, -140])
+@pytest.mark.parametrize("rows", [32, 200])
+def test_subnormal_values(rows, e):
+    """V below fp32's normal range, where the matrix core reads zeros: within the
+    rounding of the products and sums to multiples of 2^-149, one each a key at
+    most, over four partial sums."""
+    q, k, v = _inputs(rows, rows)
+    got, want = _run(q, k, v.abs() * 2.0 ** e)
+    assert float((got - want).abs().max()) <= rows * 2.0 ** -149
+    assert (got - want).norm() <= 0.02 * want.norm()
+
+
+def test_zero_columns():
+    """Zeros in V (a head padded to its width) are zeros in the result."""
+    q, k, v = _inputs(5, 300)
+    v.view(-1, NKV, D)[:, :, 100:] = 0.0
+    got, want = _run(q, k, v)
+    assert bool((got.view(-1, NH, D)[:, :, 100:] == 0).all())
+    assert (got - want).norm() <= 1e-6 * want.norm()
+
+
 @pytest.mark.parametrize("rows,stride", [(3, (1 << 22) - 4), (3, 1 << 22), (1000, 1 << 20),
                                          (1023, 1 << 20), (1025, 1 << 20)])
 def test_far_rows(rows, stride):
