@@ -353,16 +353,26 @@ hipError_t launch_wide_mode(const GemmArgs& a, hipStream_t st) {
 
 }  // namespace
 
-// Where the form is the faster one (sweep over M = 384 .. 8192 at the LM's
-// widths, both code layouts, against the 16x16x32 kernel's tiles for the same
-// shape): SiLU from 640 rows (M = 600 within 2 %, 512 row by row equal); stores
-// where the 128 x 64 tiles fill the four workgroup slots of every CU, or between
-// 1024 and 2048 rows about half of them (N = 3072, M = 1280, 480 tiles: 17.9
-// against 20.7; M = 1024, 384 tiles: 17.1 against 16.6).
+// Where the form is the faster one (swept with the weights rotated through 600 MB,
+// both code layouts, against the 16x16x32 kernel's tiles for the same shape).  SiLU
+// from 640 rows (M = 600 within 2 %, 512 row by row equal).  Stores where the 128 x
+// 64 tiles fill the four workgroup slots of every CU, or between 1024 and 2048 rows
+// about half of them (K = 1024, N = 3072, M = 1280, 480 tiles, the other kernel /
+// this one: row-major codes 20.2 / 18.3 us, tile-major 18.2 / 17.2), and where K is
+// long enough for the ring, whose three stages fill and drain for nothing below
+// (N = 8200, M = 1024, row-major: K = 128 1.46 times the other's time, 256 1.17,
+// 512 1.04; over all N from 1024 to 12000 0.98 to 1.28 times at K = 256, 0.89 to
+// 1.14 at 512), except that 512 pays from 4096 rows and columns (0.84 to 1.0, once
+// 1.05).  Below 2048 rows the other kernel's 128 x 64 tiles come out even at 1024
+// rows of 6144 columns or more (K = 1024 22.3 / 23.3 us, N = 6144; 31.3 / 32.2, 8200)
+// and over rows of more than 10240 columns (K = 768, N = 12000, M = 1536 47.3 /
+// 53.5); from K = 1536 the two are level there.
 bool wide_applies(const GemmArgs& a, GemmMode mode) {
   if (a.Kb % 4 || a.W16) return false;
   if (mode == kSiluQuant) return a.M >= 640;
   if (mode != kStore && mode != kAccumulate && mode != kDumpBlocks) return false;
+  if (a.Kb < 24 && (a.Kb < 16 || a.M < 4096 || a.N < 4096)) return false;
+  if (a.M < 2048 && a.Kb < 48 && (a.N > 10240 || (a.M < 1088 && a.N >= 6144))) return false;
   const int64_t tiles = (((int64_t)a.N + kBN - 1) / kBN) * (((int64_t)a.M + 63) / 64);
   return a.M >= 1024 && tiles >= (a.M < 2048 ? 480 : 1000);
 }
