@@ -275,11 +275,15 @@ __device__ __forceinline__ f32x16 mfma_h(h8 a, h8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
-// Workgroup id -> (n tile, m tile): XCD x (id % 8) takes the x-th contiguous
-// range of the tiles numbered n-tile-major, so its L2 holds its own weight
-// columns and every XCD gets the same number of tiles whatever n_tiles is (65
-// at the head's 8200 columns: by whole n tiles one XCD would get 2 and seven 9).
+// Workgroup id -> (n tile, m tile).  By whole n tiles (tile_of): an XCD walks its
+// eighth of the columns m tile by m tile, so the workgroups it runs at once write
+// neighbouring columns of the same rows.  Balanced: XCD x (id % 8) takes the x-th
+// contiguous range of the tiles numbered n-tile-major, so its L2 holds its own weight
+// columns and every XCD gets the same number of tiles whatever n_tiles is (65 at the
+// head's 8200 columns: by whole n tiles one XCD would get 2 and seven 9).
+template <bool BY_N>
 __device__ __forceinline__ bool f32_tile_of(int id, int n_tiles, int m_tiles, int& nt, int& mt) {
+  if constexpr (BY_N) return tile_of(id, n_tiles, nt, mt);
   const int total = n_tiles * m_tiles, per = (total + 7) >> 3;
   const int slot = id >> 3, p = (id & 7) * per + slot;
   if (slot >= per || p >= total) return false;
@@ -288,7 +292,7 @@ __device__ __forceinline__ bool f32_tile_of(int id, int n_tiles, int m_tiles, in
   return true;
 }
 
-template <int BM, int NST>
+template <int BM, int NST, bool BY_N>
 __global__ __launch_bounds__(256) void gemm_f32s_kernel(const GemmF32Args a) {
   constexpr int FM = BM / 64;                  // 32-row tiles of m per wavefront
   constexpr int FRAGS = 8 + 2 * (BM / 32);     // per stage: (tile, plane)
@@ -298,7 +302,7 @@ __global__ __launch_bounds__(256) void gemm_f32s_kernel(const GemmF32Args a) {
   const int wn = wave & 1, wm = wave >> 1;
   const int n_tiles = (a.N + 127) / 128, m_tiles = (a.M + BM - 1) / BM;
   int nt, mt;
-  if (!f32_tile_of(blockIdx.x, n_tiles, m_tiles, nt, mt)) return;  // padding workgroup
+  if (!f32_tile_of<BY_N>(blockIdx.x, n_tiles, m_tiles, nt, mt)) return;  // padding workgroup
   const int64_t Ks = a.Ks;
   const int nst = (int)Ks;
   // this wavefront's fragments of every stage: slots wave * OPS ..
@@ -492,18 +496,31 @@ hipError_t launch_rmsnorm_split(int64_t rows, int64_t cols, const float* x, cons
 
 hipError_t launch_gemm_f32(const GemmF32Args& a, hipStream_t st) {
   if (a.M <= 0 || a.N <= 0) return hipSuccess;
-  auto go = [&](auto kernel, int bm) {
-    const int64_t tiles = (((int64_t)a.N + 127) / 128) * (((int64_t)a.M + bm - 1) / bm);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(256), 0, st, a);
+  const int64_t n_tiles = ((int64_t)a.N + 127) / 128, tiles64 = n_tiles * (((int64_t)a.M + 63) / 64);
+  auto go = [&](auto kernel, int bm, bool by_n) {
+    const int64_t m_tiles = ((int64_t)a.M + bm - 1) / bm;
+    const int64_t grid = by_n ? grid_size(n_tiles, m_tiles) : 8 * ((n_tiles * m_tiles + 7) / 8);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), 0, st, a);
     return hipGetLastError();
   };
-  // 64-row tiles up to 1536 rows: more workgroups for few rows and a smaller
-  // last round (N = 8200, K = 1024, kernel us, 64 / 128 rows: M = 40 16.4 / 25.5,
-  // 300 26.0 / 29.3, 600 38.3 / 42.1, 1200 65.3 / 67.1); above, the 128-row
-  // tile's fewer LDS reads per product (M = 2000 whole call 131.7 / 125.6, 4000
-  // 240 / 232)
-  if (a.M <= 1536) return go(gemm_f32s_kernel<64, 4>, 64);
-  return go(gemm_f32s_kernel<128, 3>, 128);
+  // Balanced order and, up to 1536 rows, 64-row tiles: more workgroups for few rows
+  // and a smaller last round (N = 8200, K = 1024, the whole call with the weight
+  // planes from HBM, us, 64 / 128 rows: M = 40 29 / 35, 300 36 / 39, 600 58 / 58,
+  // 1000 82 / 85, 1536 113 / 112); above, the 128-row tile's fewer LDS reads per
+  // product (M = 2500 165 / 159, 5000 304 / 284).
+  // By whole n tiles where the output's rows are long or the products few, and the
+  // stores are what the time goes to: K <= 128 (N = 8200, K = 77, M = 5000 64 us, 72
+  // balanced; N = 20000, M = 1536 48 / 56), K <= 384 with more than 56 n tiles (N =
+  // 8200, K = 256, M = 5000 100 / 113), and more than 80 n tiles (imbalance then
+  // below 10 %; N = 20000, K = 1024: M = 300 61 / 65, 1000 135 / 161, 5000 640 / 640).
+  // In 64 rows for K <= 128 and while one round of two workgroups a CU covers
+  // the call (N = 20000, K = 1024: M = 65 34 / 41), else in 128.
+  if (a.Ks <= 8 || n_tiles > 80 || (a.Ks <= 24 && n_tiles > 56)) {
+    if (a.Ks <= 8 || a.M <= 64 || tiles64 <= 512) return go(gemm_f32s_kernel<64, 4, true>, 64, true);
+    return go(gemm_f32s_kernel<128, 3, true>, 128, true);
+  }
+  if (a.M <= 1536) return go(gemm_f32s_kernel<64, 4, false>, 64, false);
+  return go(gemm_f32s_kernel<128, 3, false>, 128, false);
 }
 
 }  // namespace ovh

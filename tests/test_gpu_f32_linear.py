@@ -27,7 +27,12 @@ def _device():
 @pytest.mark.parametrize("offset", [0, 1], ids=["aligned", "unaligned"])
 @pytest.mark.parametrize("M,N,K", [(1, 8200, 1024), (63, 130, 16), (64, 129, 48), (65, 128, 64),
                                    (130, 300, 80), (129, 1, 256), (6, 257, 512), (1536, 200, 768),
-                                   (1537, 200, 256), (2050, 131, 1024)])
+                                   (1537, 200, 256), (2050, 131, 1024),
+                                   # few products, rows of more than 80 n tiles: by whole
+                                   # n tiles, in 64 and 128 rows
+                                   (70, 1100, 128), (1600, 1100, 77), (65, 1100, 144),
+                                   (64, 10241, 160), (200, 10369, 256), (520, 10369, 256),
+                                   (520, 10240, 256), (1537, 10241, 130)])
 def test_linear_f32_edges(M, N, K, offset):
     import ovnative_amd as ov
     g = torch.Generator().manual_seed(M + N + K)
