@@ -236,6 +236,10 @@ int64_t workgroups(int64_t M, int64_t N, int cols) {
   return (M + kRows - 1) / kRows * ((N + cols - 1) / cols);
 }
 
+bool vec4_rows(const float* A, const DeviceWeight& w) {
+  return w.K % 4 == 0 && ((uintptr_t)A & 15u) == 0;
+}
+
 template <int COLS, int KBM>
 hipError_t launch_small(int64_t M, const float* A, const DeviceWeight& w, float* C, int64_t ldc,
                         bool add, hipStream_t st) {
@@ -245,7 +249,7 @@ hipError_t launch_small(int64_t M, const float* A, const DeviceWeight& w, float*
                        A, w.q, w.scale, C, ldc);
     return hipGetLastError();
   };
-  const bool vec4 = w.K % 4 == 0 && ((uintptr_t)A & 15u) == 0;
+  const bool vec4 = vec4_rows(A, w);
   if (add)
     return vec4 ? go(linear_small_kernel<COLS, KBM, true, true>)
                 : go(linear_small_kernel<COLS, KBM, true, false>);
@@ -260,12 +264,18 @@ hipError_t launch_small(int64_t M, const float* A, const DeviceWeight& w, float*
 // 9.7 / 10.9, at 1024 11.3 / 10.6; 128 columns (one a CU) M = 333, N = 1501
 // (252 workgroups) 7.9 / 10.6, at 384 12.1 / 10.7.  K = 2048, 32 columns (one a CU):
 // M = 40, N = 1024 8.4 / 10.6, at 416 workgroups 15.8 / 10.9.  K = 3072: 12.0 / 10.7
-// at 96 workgroups (the row quantisation alone is 1.5 us), not taken.
-int small_cols(int64_t M, const DeviceWeight& w) {
+// at 96 workgroups (the row quantisation alone is 1.5 us), not taken.  Rows loaded
+// value by value (not VEC4) take four times the loads, and long ones not two
+// workgroups a CU for the time of one: K = 1001, N = 1000, 32 columns, 224 workgroups
+// 8.2 / 10.7, 320 11.8 / 10.3 (128 columns, 80 workgroups, 9.5), 128 columns at 240
+// workgroups 9.7 / 10.7, at 256 10.9 / 10.6 (where K has a 128-k tail the two launches
+// are slower: K = 850 13.4 of them); K = 250, 512 workgroups 7.6 / 10.6.
+int small_cols(int64_t M, const DeviceWeight& w, bool vec4) {
   if (w.Kb > 64) return 0;
   if (w.Kb > 32) return workgroups(M, w.N, 32) <= 256 ? 32 : 0;
-  if (workgroups(M, w.N, 32) <= 512) return 32;
-  return workgroups(M, w.N, 128) <= 256 ? 128 : 0;
+  const bool light = vec4 || w.Kb <= 24;
+  if (workgroups(M, w.N, 32) <= (light ? 512 : 256)) return 32;
+  return workgroups(M, w.N, 128) <= (light || w.Kb % 4 ? 256 : 240) ? 128 : 0;
 }
 
 }  // namespace
@@ -276,12 +286,12 @@ bool linear_small_applies(int64_t M, const float* A, const DeviceWeight& w, cons
   // C written while other workgroups still read A: not where they overlap
   const float *a1 = A + M * w.K, *c1 = C + (M - 1) * ldc + w.N;
   if (C < a1 && A < c1) return false;
-  return small_cols(M, w) != 0;
+  return small_cols(M, w, vec4_rows(A, w)) != 0;
 }
 
 hipError_t launch_linear_small(int64_t M, const float* A, const DeviceWeight& w, float* C,
                                int64_t ldc, bool add, hipStream_t st) {
-  const int cols = small_cols(M, w);
+  const int cols = small_cols(M, w, vec4_rows(A, w));
   if (cols == 32 && w.Kb <= 32) return launch_small<32, 32>(M, A, w, C, ldc, add, st);
   if (cols == 32 && w.Kb <= 64) return launch_small<32, 64>(M, A, w, C, ldc, add, st);
   if (cols == 128 && w.Kb <= 32) return launch_small<128, 32>(M, A, w, C, ldc, add, st);

@@ -57,6 +57,15 @@ def test_one_launch_linear(M, N, K, offset):
                 ov.linear_q(aq, asc, w, C=C0.clone(), accumulate=True))
 
 
+# rows loaded value by value, on both sides of the lines between 32 columns, 128
+# columns and two launches
+@pytest.mark.parametrize("M,N,K", [(128, 1024, 1001), (129, 1024, 1001), (480, 1024, 1001),
+                                   (481, 1024, 1001), (512, 1024, 850), (513, 1024, 850),
+                                   (256, 1024, 767), (257, 1024, 767)])
+def test_one_launch_linear_odd_rows(M, N, K):
+    test_one_launch_linear(M, N, K, 0)
+
+
 def test_leading_dimension_and_overlap():
     """Columns past N of a wider C stay as they are; C over A still gives
     A + linear(A) of the old A."""
