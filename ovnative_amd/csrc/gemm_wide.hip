@@ -379,7 +379,10 @@ bool wide_applies(const GemmArgs& a, GemmMode mode) {
 
 // 64-row tiles, except for the SiLU form from 4096 rows, where its longer
 // epilogue gains from the larger tile (M = 4096 72.7 against 69.1 us, 2048 39.3
-// against 38.4, 3000 55.5 against 56.5, whose 1152 tiles end in a half-full round).
+// against 38.4, 3000 55.5 against 56.5, whose 1152 tiles end in a half-full round),
+// as long as there are enough of those tiles (64- / 128-row tiles, K = 1024: N = 128,
+// M = 4096, 32 tiles 11.8 / 17.9; N = 896, M = 5000, 280 tiles 19.3 / 23.9, M = 8192,
+// 448 tiles 25.2 / 25.1).
 hipError_t launch_gemm_wide(const GemmArgs& a, GemmMode mode, hipStream_t st) {
   switch (mode) {
     case kStore: return launch_wide_mode<64, kStore>(a, st);
@@ -387,8 +390,9 @@ hipError_t launch_gemm_wide(const GemmArgs& a, GemmMode mode, hipStream_t st) {
     case kDumpBlocks: return launch_wide_mode<64, kDumpBlocks>(a, st);
     case kSiluQuant:
       if (a.N % 128 || !a.hq || !a.hsc || a.hKp < a.N / 2) return hipErrorInvalidValue;
-      return a.M >= 4096 ? launch_wide_mode<128, kSiluQuant>(a, st)
-                         : launch_wide_mode<64, kSiluQuant>(a, st);
+      return a.M >= 4096 && a.N / 128 * (((int64_t)a.M + 127) / 128) >= 448
+                 ? launch_wide_mode<128, kSiluQuant>(a, st)
+                 : launch_wide_mode<64, kSiluQuant>(a, st);
     default: return hipErrorInvalidValue;
   }
 }

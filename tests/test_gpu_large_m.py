@@ -175,3 +175,18 @@ def test_silu_epilogue_bounds(M, reach):
     hq, hsc = ov.silu_gate_linear(aq, asc, ov.gate_up_weight(wg, wu))
     assert torch.equal(hq, want_q)
     assert same(hsc, want_s)
+
+
+# both sides of the 128-row tile's line (448 of them): 416, 448, 528 and 231
+@pytest.mark.parametrize("M,I", [(4096, 832), (4096, 896), (4097, 1024), (4095, 448)])
+def test_silu_tile_rows(M, I):
+    import ovnative_amd as ov
+    rng = np.random.default_rng(I)
+    K = 256
+    (wg, _, _), (wu, _, _) = _weight(rng, I, K), _weight(rng, I, K)
+    aq, asc = ov.s8_nk_quantize(torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32))
+                                .cuda())
+    want_q, want_s = ov.silu_mul_quantize(ov.linear_q(aq, asc, wg), ov.linear_q(aq, asc, wu))
+    hq, hsc = ov.silu_gate_linear(aq, asc, ov.gate_up_weight(wg, wu))
+    assert torch.equal(hq, want_q)
+    assert same(hsc, want_s)
