@@ -41,23 +41,27 @@ hipError_t launch_rope_tables(int64_t rows, const int64_t* pos, int D, float the
 
 // ---------------------------------------------------------------------------
 // Per-head RMSNorm then RoPE, cpp/src/backend/cpu/ops_cpu.cpp:266-318
-// (norm_rope_head_avx2).  One wavefront per (row, head); lane t < D/2 owns the
-// rotation pair (t, t + D/2).  The sum of squares reproduces the reference's
-// 8-lane fma accumulator: chain j takes elements j, j+8, ... in order, and the
-// 8 chains are added left to right, so the norm scale is the reference's bits.
-// Lane t < D/2 of the wavefront returns the normalised, rotated pair (t, t + D/2)
-// of the head vector v in (oa, ob); the other lanes return false.
-template <int D>
-__device__ __forceinline__ bool norm_rope_pair(const float* __restrict__ v,
-                                               const float* __restrict__ w,
-                                               const float* __restrict__ cos_row,
-                                               const float* __restrict__ sin_row, float eps,
-                                               int lane, float& oa, float& ob) {
-  constexpr int half = D / 2;
+// (norm_rope_head_avx2), for heads of 64.  One wavefront per (row, head); lane t <
+// 32 owns the rotation pair (t, t + 32).  The sum of squares reproduces the
+// reference's 8-lane fma accumulator: chain j takes elements j, j+8, ... in order,
+// and the 8 chains are added left to right, so the norm scale is the reference's
+// bits.
+__global__ __launch_bounds__(256) void qk_norm_rope_64_kernel(
+    float* __restrict__ q, float* __restrict__ k, const float* __restrict__ qw,
+    const float* __restrict__ kw, int64_t rows, int n_heads, int n_kv_heads,
+    const float* __restrict__ cos_tab, const float* __restrict__ sin_tab, float eps) {
+  constexpr int D = 64, half = D / 2;
+  const int lane = threadIdx.x & 63;
+  const int heads = n_heads + n_kv_heads;
+  const int64_t task = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (task >= rows * heads) return;  // whole wavefront leaves together
+  const int64_t r = task / heads;
+  const int h = (int)(task - r * heads);
+  float* v = h < n_heads ? q + (r * n_heads + h) * D : k + (r * n_kv_heads + (h - n_heads)) * D;
+  const float* const w = h < n_heads ? qw : kw;
   const bool own = lane < half;
   const float a = own ? v[lane] : 0.f;
   const float b = own ? v[lane + half] : 0.f;
-
   // Chain j = lane % 8 (lanes 8.. compute copies that are not used).
   const int j = lane & 7;
   float s = 0.f;
@@ -71,39 +75,12 @@ __device__ __forceinline__ bool norm_rope_pair(const float* __restrict__ v,
 #pragma unroll
   for (int c = 1; c < 8; ++c) sum = __fadd_rn(sum, __shfl(s, c));
   const float scale = __fdiv_rn(1.f, sqrt_rn(__fadd_rn(__fdiv_rn(sum, (float)D), eps)));
-  if (!own) return false;
-  const float c = cos_row[lane], sn = sin_row[lane];
+  if (!own) return;
+  const float c = cos_tab[r * half + lane], sn = sin_tab[r * half + lane];
   const float na = __fmul_rn(__fmul_rn(a, scale), w[lane]);
   const float nb = __fmul_rn(__fmul_rn(b, scale), w[lane + half]);
-  oa = fmaf(na, c, -__fmul_rn(nb, sn));
-  ob = fmaf(na, sn, __fmul_rn(nb, c));
-  return true;
-}
-
-template <int D>
-__global__ __launch_bounds__(256) void qk_norm_rope_kernel(float* __restrict__ q,
-                                                           float* __restrict__ k,
-                                                           const float* __restrict__ qw,
-                                                           const float* __restrict__ kw,
-                                                           int64_t rows, int n_heads,
-                                                           int n_kv_heads,
-                                                           const float* __restrict__ cos_tab,
-                                                           const float* __restrict__ sin_tab,
-                                                           float eps) {
-  constexpr int half = D / 2;
-  const int lane = threadIdx.x & 63;
-  const int heads = n_heads + n_kv_heads;
-  const int64_t task = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (task >= rows * heads) return;  // whole wavefront leaves together
-  const int64_t r = task / heads;
-  const int h = (int)(task - r * heads);
-  float* v = h < n_heads ? q + (r * n_heads + h) * D : k + (r * n_kv_heads + (h - n_heads)) * D;
-  float oa, ob;
-  if (!norm_rope_pair<D>(v, h < n_heads ? qw : kw, cos_tab + r * half, sin_tab + r * half, eps,
-                         lane, oa, ob))
-    return;
-  v[lane] = oa;
-  v[lane + half] = ob;
+  v[lane] = fmaf(na, c, -__fmul_rn(nb, sn));
+  v[lane + half] = fmaf(na, sn, __fmul_rn(nb, c));
 }
 
 // D = 128 with 8 lanes per head vector (norm_rope_lanes8): the chains run in
@@ -141,7 +118,7 @@ hipError_t launch_qk_norm_rope(float* q, float* k, const float* qw, const float*
     hipLaunchKernelGGL(qk_norm_rope_lanes8_kernel, dim3((unsigned)((tasks + 31) / 32)), dim3(256),
                        0, st, q, k, qw, kw, rows, n_heads, n_kv_heads, cos_tab, sin_tab, eps);
   else
-    hipLaunchKernelGGL(qk_norm_rope_kernel<64>, dim3((unsigned)((tasks + 3) / 4)), dim3(256), 0,
+    hipLaunchKernelGGL(qk_norm_rope_64_kernel, dim3((unsigned)((tasks + 3) / 4)), dim3(256), 0,
                        st, q, k, qw, kw, rows, n_heads, n_kv_heads, cos_tab, sin_tab, eps);
   return hipGetLastError();
 }
