@@ -199,8 +199,8 @@ hipError_t launch_gemm_grouped(const GemmGroups& gg, GemmMode mode, hipStream_t 
 // M <= 128, K a multiple of 1024 up to 3072, int8 form, one output slice.
 bool skinny_applies(const GemmGroups& gg);
 hipError_t launch_gemm_skinny(const GemmGroups& gg, GemmMode mode, hipStream_t st);
-// The large-M form (gemm_wide.hip): block products on the f16 matrix core, the
-// int8 operands widened on their way into LDS; the same bits.
+// The large-M form (gemm_wide.hip): 32x32x32 int8 products, operands staged by DMA
+// through a three-stage ring; the same bits.
 bool wide_applies(const GemmArgs& a, GemmMode mode);
 hipError_t launch_gemm_wide(const GemmArgs& a, GemmMode mode, hipStream_t st);
 // Rows from which the GEMMs take the f16-operand form (GemmArgs::W16/aq16);

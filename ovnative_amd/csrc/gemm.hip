@@ -1361,7 +1361,8 @@ hipError_t launch_gemm_grouped(const GemmGroups& in, GemmMode mode, hipStream_t 
   int64_t max_m = 0;
   for (int g = 0; g < in.n; ++g) {
     const GemmArgs& a = in.args[g];
-    if (a.Kb % 4 || a.W16 || a.M <= 0) return hipErrorInvalidValue;
+    // (the grouped kernels read row-major codes)
+    if (a.Kb % 4 || a.W16 || a.a_tiled || a.M <= 0) return hipErrorInvalidValue;
     max_m = a.M > max_m ? a.M : max_m;
   }
   // The members with the longest K loops first: their workgroups are
