@@ -313,7 +313,12 @@ int ovh_qk_norm_rope(float* q, float* k, const float* qw, const float* kw, int64
  * h / (n_heads / n_kv_heads)), out = softmax(q k^T * scale + bias) v in fp32,
  * zeros for a fully masked row (max < -1e29).  q/out rows have stride q_stride
  * / out_stride, k/v rows kv_stride (elements).  head_dim 128.  segs is HOST
- * memory (any count; launched 32 segments at a time). */
+ * memory (any count; launched 32 segments at a time).
+ * The products are those of three bf16 parts a value, which carry them to 2^-24
+ * over fp32's range (the results are no further from float64 than with fp32
+ * products); 32-row tiles with values that do not split (not finite, or beyond
+ * what the parts' range allows) are computed with fp32 products instead, at up to
+ * 1.6 times those products' time. */
 int ovh_attention(const OvhAttnSegment* segs, int n_segs, int n_heads, int n_kv_heads,
                   int head_dim, const float* q, int64_t q_stride, const float* k, const float* v,
                   int64_t kv_stride, float scale, float* out, int64_t out_stride, void* stream);
@@ -322,7 +327,10 @@ int ovh_attention(const OvhAttnSegment* segs, int n_segs, int n_heads, int n_kv_
  * time of the fp32 form).  No reference counterpart beyond ovh_attention's.
  * |k| and |v| must stay below 65504 (OV_ERR_INVALID_ARG otherwise); strides a
  * multiple of 8, kv_off a whole number of rows, at most 32 segments.  Allocates
- * its split workspace stream-ordered and synchronises the stream. */
+ * its split workspace stream-ordered and synchronises the stream.  That workspace
+ * and ovh_linear_f32's come from a memory pool of the library's own, one per device,
+ * which keeps up to 256 MB of device memory from call to call until the process
+ * ends.  Any number of threads and streams may call at once. */
 int ovh_attention_split(const OvhAttnSegment* segs, int n_segs, int n_heads, int n_kv_heads,
                         int head_dim, const float* q, int64_t q_stride, const float* k,
                         const float* v, int64_t kv_stride, float scale, float* out,

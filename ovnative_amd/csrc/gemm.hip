@@ -1393,6 +1393,13 @@ hipError_t launch_gemm(const GemmArgs& a, GemmMode mode, hipStream_t st) {
   // M >= 512 keep a 128x64 tile (wave 64x32: one weight fragment feeds two
   // MFMAs), mid-size ones 64x64, and skinny M or N = 1024 one-wave 32x32 tiles,
   // which give the most wavefronts for the few output tiles there are.
+  // The rings' figures below are of tile-major codes (the runner's).  Row-major ones
+  // come by rows in the pipelined tiles since; the same choices as calls, cold
+  // weights, chosen / the others named there, us row-major and tile-major: N = 1024,
+  // K = 3072, M = 128 8.4 / 9.7 and 7.9 / 9.8 (4-block stages); M = 300 9.6 / 11.2 and
+  // 9.3 / 11.0; M = 600 11.1 / 12.4 / 12.1 and 10.7 / 12.5 / 11.9; M = 1200 17.7 / 17.1
+  // and 17.2 / 16.6; N = 4096, K = 1024, M = 600 12.7 / 12.9 and 12.7 / 15.9, M = 1200
+  // 20.9 / 21.9 and 20.9 / 20.7.  (A call takes 7.7 at least: K = 2048 shows less.)
   const int64_t M = a.M, N = a.N;
   // Stage loop: the software pipeline pays where a wavefront holds few output
   // tiles (32x32 and 64x32 workgroups, the SiLU tile at M = 600: 17.7 vs

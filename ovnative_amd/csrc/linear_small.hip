@@ -26,7 +26,8 @@ constexpr int kRows = 16, kWaves = 8, kThreads = 64 * kWaves;
 // worked out by one of its 8 lanes (lane p for pass p), without the general
 // division's exponent scaling: 127 / amax by one Newton step and one residual
 // correction, amax / 127 by one correction, both equal to the IEEE quotient for
-// every significand (checked over all 2^23) while amax is in [2^-100, 2^120].
+// every significand while amax is in [2^-100, 2^120] (all 2^23 of them, for a
+// reciprocal one unit off either way: tests/short_quotients.cpp).
 // Rows with a NaN or an amax outside that range (zero is inside) go the general
 // way.
 template <int P>

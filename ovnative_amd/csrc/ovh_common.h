@@ -212,10 +212,11 @@ __device__ __forceinline__ float silu_up_lane(float g, float u) {
 //  * the clamp as one med3 (a NaN in g gives NaN either way);
 //  * rint(y) as (y + 1.5 2^23) - 1.5 2^23 (|y| <= 127), whose low bits are also
 //    the exponent the scale 2^n needs;
-//  * the quotient g / d without the exponent scaling of the general division:
-//    the same reciprocal refinement and two residual corrections, correctly
+//  * the quotient g / d without the exponent scaling of the general division: one
+//    Newton step on the reciprocal and two corrections of the quotient by its
+//    exact residual (P. Markstein, IBM J. Res. Dev. 34 (1990) 111), correctly
 //    rounded where nothing in it over- or underflows: d in [1, 2^97) (g >= -66)
-//    and 2^-100 <= |g| <= 2^60.
+//    and 2^-100 <= |g| <= 2^60 (tests/short_quotients.cpp).
 // Where a g is outside that range (zero included) every lane of the wavefront
 // takes silu_up_lane.  (Gate/up at M = 16384, N = 6144, K = 1024, together with
 // the tile of gemm_wide.hip: 349 -> 300 us a launch.)
