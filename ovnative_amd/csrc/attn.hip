@@ -340,7 +340,7 @@ __device__ __forceinline__ void attention_f32_body(const AttnArgs& args, const A
 // instead of 70.
 // K's next block is fetched in halves: all of it beside all of V spilled 164 B.
 // 16 heads, fp32 products -> these: the call with 2 segments of 700 rows 105 ->
-// 69 us, 16 x 600 rows 522 -> 352, masked 595 -> 438, 2 x 200 17.4 -> 17.2, 33 rows
+// 69 us, 16 x 600 rows 522 -> 350, masked 595 -> 432, 2 x 200 17.4 -> 17.0, 33 rows
 // 15 (either); error against 64 bits 5.0e-7 -> 4.1e-7 of the result's norm (700
 // rows).  Rows are addressed with 32-bit offsets (24-bit products): 64-bit ones
 // per lane took 2 x 700 rows 4 us longer.
@@ -362,14 +362,15 @@ __device__ __forceinline__ Parts split3(const float (&x)[8]) {
   for (int i = 0; i < 4; ++i) {
     f32x2 v = {x[2 * i], x[2 * i + 1]};
 #pragma unroll
-    for (int part = 0; part < 3; ++part) {
+    for (int part = 0; part < 2; ++part) {
       const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, b2));
       d[part][i] = (int)u;
-      if (part < 2) {
-        v[0] = __fsub_rn(v[0], __uint_as_float(u << 16));
-        v[1] = __fsub_rn(v[1], __uint_as_float(u & 0xffff0000u));
-      }
+      v[0] = __fsub_rn(v[0], __uint_as_float(u << 16));
+      v[1] = __fsub_rn(v[1], __uint_as_float(u & 0xffff0000u));
     }
+    // lo is a bf16 already: its upper half (V_PERM_B32; V_CVT_PK_BF16_F32 takes twice
+    // the time)
+    d[2][i] = (int)__builtin_amdgcn_perm(__float_as_uint(v[1]), __float_as_uint(v[0]), 0x07060302u);
   }
   return Parts{__builtin_bit_cast(b8, d[0]), __builtin_bit_cast(b8, d[1]),
                __builtin_bit_cast(b8, d[2])};
@@ -421,10 +422,11 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qt
   const char* const kb = reinterpret_cast<const char*>(args.k + seg.kv_off + (int64_t)kvh * kAttnD);
   const char* const vb = reinterpret_cast<const char*>(args.v + seg.kv_off + (int64_t)kvh * kAttnD);
   // A row's bytes from the segment's first: 24-bit factors and a 32-bit product, or
-  // the fp32 products below, which count in 64 bits.
-  const uint32_t row_bytes = 4 * (uint32_t)args.kv_stride;
+  // the fp32 products below, which count in 64 bits (then only the first row is
+  // loaded here: a branch around these loads would wait for them where it ends).
   const bool small = S < 1 << 24 && args.kv_stride < 1 << 22 &&
                      4 * args.kv_stride * S < (int64_t)0xffff0000;
+  const uint32_t row_bytes = small ? 4 * (uint32_t)args.kv_stride : 0;
   auto row_at = [&](int t) __attribute__((always_inline)) {
     return (uint32_t)__umul24((uint32_t)min(t, S - 1), row_bytes);
   };
@@ -448,10 +450,8 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qt
           vb + (row_at(t0 + 8 * (i >> 2) + 4 * hf + (i & 3)) + 16 * r32));
   };
   const int nblk = (S + kAttnK - 1) / kAttnK;
-  if (small) {
-    load_k(min(wave, nblk - 1) * kAttnK, 0);
-    load_k(min(wave, nblk - 1) * kAttnK, 1);
-  }
+  load_k(min(wave, nblk - 1) * kAttnK, 0);
+  load_k(min(wave, nblk - 1) * kAttnK, 1);
   // ---- Q: 16 values of a row per thread, split into LDS
   const float as = fabsf(args.scale), q_max = 0x1p90f / fmaxf(as, 1.f);
   bool odd = !small || !(as >= 0x1p-30f && as <= 0x1p60f);
@@ -538,7 +538,7 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qt
     psum = __fadd_rn(psum, __shfl_xor(psum, 32));
     float alpha = 1.f;
     if (__any(up && m_run > -INFINITY)) {  // uniform; before, sum and output are 0
-      alpha = expf(m_run - m_ref);
+      alpha = __fmul_rn(exp_p64(m_run - m_ref), 0x1p-64f);
       if (hf == 0) alpha_s[wave][r32] = alpha;
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -601,7 +601,7 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qt
   float f[kAttnWaves], L = 0.f;
 #pragma unroll
   for (int w = 0; w < kAttnWaves; ++w) {
-    f[w] = mstat[w][qi] == -INFINITY ? 0.f : expf(mstat[w][qi] - M);
+    f[w] = mstat[w][qi] == -INFINITY ? 0.f : __fmul_rn(exp_p64(mstat[w][qi] - M), 0x1p-64f);
     L = fmaf(lstat[w][qi], f[w], L);
   }
   const float inv = __fdiv_rn(1.f, L);
@@ -624,21 +624,24 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(AttnArgs args, int qt
       zero |= ov[j + c] == 0.f && M >= -1e29f;
     }
   }
-  odd = __syncthreads_or(odd || !(nan == 0.f));
-  // A zero: there is nothing in the column, or only values below 2^-126, which the
-  // matrix core takes for zeros.  The segment's V tells.
-  if (!odd && __syncthreads_or(zero)) {
-    bool tiny = false;
-    for (int t = threadIdx.x >> 5; t < S; t += 8) {
-      const f32x4 x = *reinterpret_cast<const f32x4*>(vb + (row_at(t) + 16 * (threadIdx.x & 31)));
+  odd |= !(nan == 0.f);
+  if (__syncthreads_or(odd || zero)) {
+    odd = __syncthreads_or(odd);
+    // A zero: there is nothing in the column, or only values below 2^-126, which the
+    // matrix core takes for zeros.  The segment's V tells.
+    if (!odd) {
+      bool tiny = false;
+      for (int t = threadIdx.x >> 5; t < S; t += 8) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(vb + (row_at(t) + 16 * (threadIdx.x & 31)));
 #pragma unroll
-      for (int c = 0; c < 4; ++c) tiny |= x[c] != 0.f && fabsf(x[c]) < 0x1p-126f;
+        for (int c = 0; c < 4; ++c) tiny |= x[c] != 0.f && fabsf(x[c]) < 0x1p-126f;
+      }
+      odd = __syncthreads_or(tiny);
     }
-    odd = __syncthreads_or(tiny);
-  }
-  if (odd) {
-    attention_f32_body(args, seg, h, q0, part, mstat, lstat, alpha_s);
-    return;
+    if (odd) {
+      attention_f32_body(args, seg, h, q0, part, mstat, lstat, alpha_s);
+      return;
+    }
   }
   if (q0 + qi >= S) return;
   float* const dst =
