@@ -270,7 +270,7 @@ __global__ __launch_bounds__(64) void rmsnorm_split_rows_kernel(const float* __r
 // set between the products of stage s, one read after each product; stage s's
 // slot is then free at the barrier that publishes stage s + 1.  M = 600,
 // N = 8200, K = 1024: 47.2 -> 40.9 us (640 -> 739 TFLOP/s of f16 products)
-// with the planes in the last-level cache, 47.8 -> 47.4 from HBM.
+// with the planes in the last-level cache, 47.1 -> 45.0 from HBM.
 __device__ __forceinline__ f32x16 mfma_h(h8 a, h8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
@@ -503,18 +503,19 @@ hipError_t launch_gemm_f32(const GemmF32Args& a, hipStream_t st) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), 0, st, a);
     return hipGetLastError();
   };
+  // (Whole calls, us, the weight planes from HBM: 600 MB of them in turn.)
   // Balanced order and, up to 1536 rows, 64-row tiles: more workgroups for few rows
-  // and a smaller last round (N = 8200, K = 1024, the whole call with the weight
-  // planes from HBM, us, 64 / 128 rows: M = 40 29 / 35, 300 36 / 39, 600 58 / 58,
-  // 1000 82 / 85, 1536 113 / 112); above, the 128-row tile's fewer LDS reads per
-  // product (M = 2500 165 / 159, 5000 304 / 284).
+  // and a smaller last round (N = 8200, K = 1024, 64 / 128 rows: M = 40 27.7 / 35.8,
+  // 300 37.9 / 38.0, 600 52.5 / 53.4, 1000 75.6 / 75.9, 1536 103 / 102); above, the
+  // 128-row tile's fewer LDS reads per product (M = 2000 136 / 126, 5000 294 / 278).
   // By whole n tiles where the output's rows are long or the products few, and the
-  // stores are what the time goes to: K <= 128 (N = 8200, K = 77, M = 5000 64 us, 72
-  // balanced; N = 20000, M = 1536 48 / 56), K <= 384 with more than 56 n tiles (N =
-  // 8200, K = 256, M = 5000 100 / 113), and more than 80 n tiles (imbalance then
-  // below 10 %; N = 20000, K = 1024: M = 300 61 / 65, 1000 135 / 161, 5000 640 / 640).
-  // In 64 rows for K <= 128 and while one round of two workgroups a CU covers
-  // the call (N = 20000, K = 1024: M = 65 34 / 41), else in 128.
+  // stores are what the time goes to (by n / balanced, in 64 rows for K <= 128, else
+  // 128): K <= 128 (N = 8200, K = 77, M = 5000 61 / 83; N = 20000, M = 1536 47 / 64), K
+  // <= 384 with more than 56 n tiles (N = 8200, K = 256, M = 5000 94 / 115), and more
+  // than 80 n tiles, the imbalance then below 10 % (N = 20000, K = 1024: M = 300 56 /
+  // 56, 1000 136 / 139, 5000 605 / 623).  There 64 rows while one round of two
+  // workgroups a CU covers the call (64 / 128 rows: M = 65 33 / 39, 129 41 / 47, 300
+  // 63 / 56).
   if (a.Ks <= 8 || n_tiles > 80 || (a.Ks <= 24 && n_tiles > 56)) {
     if (a.Ks <= 8 || a.M <= 64 || tiles64 <= 512) return go(gemm_f32s_kernel<64, 4, true>, 64, true);
     return go(gemm_f32s_kernel<128, 3, true>, 128, true);
