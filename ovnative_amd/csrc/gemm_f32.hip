@@ -269,7 +269,7 @@ __global__ __launch_bounds__(64) void rmsnorm_split_rows_kernel(const float* __r
 // its 2.5 PFLOP/s).  So stage s + 1's fragments are read into a second register
 // set between the products of stage s, one read after each product; stage s's
 // slot is then free at the barrier that publishes stage s + 1.  M = 600,
-// N = 8200, K = 1024: 47.2 -> 40.9 us (640 -> 739 TFLOP/s of f16 products)
+// N = 8200, K = 1024: 47.5 -> 39.4 us (636 -> 767 TFLOP/s of f16 products)
 // with the planes in the last-level cache, 47.1 -> 45.0 from HBM.
 __device__ __forceinline__ f32x16 mfma_h(h8 a, h8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);

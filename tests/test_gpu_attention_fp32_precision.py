@@ -69,6 +69,23 @@ def _two_keys(scores, values):
     return q.view(rows, -1), k.view(rows, -1), v.view(rows, -1)
 
 
+def test_products():
+    """Scores of one product each, of significands whose parts cut off lose most (7.8
+    units of 2^-24) and of random ones: e^(-16 x y) within the product's error (the
+    dropped parts' 2^-24 of it and its rounding's 2^-24, absolute in the exponent) and
+    the exponential's."""
+    g = torch.Generator().manual_seed(1)
+    worst = torch.tensor([1 + 2.0 ** -7 - 2.0 ** -23, 1 + (2.0 ** 16 - 1) * 2.0 ** -23,
+                          1 + 2.0 ** -7 - 2.0 ** -16, 1 + 2.0 ** -8 + 2.0 ** -16])
+    x = torch.cat([worst, 1 + torch.rand((28,), generator=g)]).cuda()
+    for y in x.tolist()[:8]:
+        q, k, v = _two_keys(-16 * x[:, None].expand(-1, NH), (0.0, 1.0))
+        k.view(-1, NKV, D)[1, :, 0] = y
+        got, want = _run(q, k, v, scale=1.0)
+        product = 16 * x[:, None].double() * y
+        assert bool(((got - want).abs() / want <= 2.0 ** -23 * product + 3.6e-7).all()), y
+
+
 @pytest.mark.parametrize("top", [0.0, -4.0, -10.0, -20.0, -40.0])
 def test_probabilities(top):
     """e^x, x down to -60, to fp32's precision: the hardware's 2^y is good to one
